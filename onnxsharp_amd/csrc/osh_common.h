@@ -194,7 +194,8 @@ long long winograd_max_pixels();
 bool nchwc_enabled();
 
 // DynamicQuantizeMatMul pipeline (0 = min/max launch then one fused
-// quantize + GEMM launch, 1 = min/max, quantize and GEMM as three launches).
+// quantize + GEMM launch, three launches for large products; 1 = always
+// min/max, quantize and GEMM as three launches).
 int dqmm_variant();
 // Kernel launches of the calling thread's last DynamicQuantizeMatMul (2 or 3).
 int dqmm_last_launches();

@@ -5,16 +5,16 @@
 // (QuantizedMatMulOps.cs:280-335) and the zero-point identity of PackedInt8Weights
 // (src/OnnxSharp/Kernels/Int8Gemm.cs:66-70).
 //
-// Pipeline (three launches, all on the caller's stream; by default 2 and 3
-// run as one launch, dqmm_fused_kernel):
+// Pipeline (three launches, all on the caller's stream; smaller products run 2
+// and 3 as one launch, dqmm_fused*_kernel or, up to 16 rows, dqmm_skinny_kernel):
 //   1. dqmm_minmax_kernel   grid-stride min/max of A (0 included, NaN skipped) into per-block
 //                           partials.
 //   2. dqmm_quantize_kernel every block reduces the partials to scale = (max-min)/255 (1 if
 //                           not > 0), zp = clamp(rne(-min/scale)), inv = 1/scale -- single IEEE
 //                           ops, no contraction -- then q = clamp(rne(x*inv) + zp, 0, 255); stores
-//                           a'' = q - 128 as s8 in the MFMA operand layout, the per-row sums of
-//                           a'', and a per-row flag for x*inv = NaN (the reference's q is then
-//                           NaN and its whole output row is NaN).
+//                           a'' = q - 128 as s8 in the MFMA operand layout and a per-row flag
+//                           for x*inv = NaN (the reference's q is then NaN and its whole
+//                           output row is NaN).
 //   3. dqmm_gemm_kernel     v_mfma_i32_32x32x32_i8 over a'' x w'' (both s8), then the exact
 //                           integer correction
 //                             acc = sum a''w'' + off_j*rowsum_i + alpha*colsum_j + K*alpha*off_j
@@ -27,6 +27,7 @@
 // lane l carries row/column (l & 31) of the tile and k = kstep*32 + 16*(l >> 5) + byte.
 // A and B use the same k assignment, so the MFMA pairs matching k regardless of the
 // hardware's internal k order.
+#include <type_traits>
 #include "osh_common.h"
 
 using namespace osh;
@@ -35,7 +36,7 @@ namespace osh {
 
 constexpr int DQ_MINMAX_BLOCKS = 256;
 constexpr int DQ_THREADS = 256;
-constexpr int DQ_KC = 16;  // k-steps of 32 per GEMM load chunk (K = 512 in one chunk)
+constexpr int DQ_MMU = 4;  // 16-byte loads a thread of the min/max launch has in flight
 
 struct DqScratch {  // layout of the caller's scratch buffer
     float partial_min[DQ_MINMAX_BLOCKS];
@@ -45,7 +46,7 @@ struct DqScratch {  // layout of the caller's scratch buffer
     float inv;
     int alpha;  // a - a_zp = a'' + alpha for the packed a'' (128 - zp for quantized u8)
     int pad[60];
-    // followed by: int rowsum[mpad]; int rownan[mpad]; int8 a_packed[mpad * kpad]
+    // followed by: int rownan[mpad]; int spare[mpad]; int8 a_packed[mpad * kpad]
 };
 
 __host__ __device__ static inline int pad32(int v) { return (v + 31) & ~31; }
@@ -83,27 +84,41 @@ __device__ void block_minmax(float &lo, float &hi) {
     }
 }
 
+// `zero` (zero_n ints, may be none): the NaN flags the quantize launch raises,
+// cleared here so that the scratch needs no initialisation.
 __global__ __launch_bounds__(DQ_THREADS) void dqmm_minmax_kernel(const float *__restrict__ a, long long n,
-                                                                  DqScratch *__restrict__ sc) {
+                                                                  DqScratch *__restrict__ sc, int *__restrict__ zero,
+                                                                  int zero_n) {
     float lo = 0.f, hi = 0.f;  // 0 is always inside the range (Quantization.cs:115-116)
-    long long stride = (long long)gridDim.x * blockDim.x;
+    const long long stride = (long long)gridDim.x * blockDim.x;
     // XCD-banded block ids: the workgroups of one XCD read one contiguous band
     // of A, which the fused kernel's workgroups on the same XCD (banded the
     // same way, row tiles first) then find in that XCD's L2.  Min and max are
     // exact in any order, so the partials' assignment does not matter.
-    long long i = (long long)xcd_band(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const long long i = (long long)xcd_band(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    for (long long z = (long long)blockIdx.x * blockDim.x + threadIdx.x; z < zero_n; z += stride) zero[z] = 0;
     // 16-byte loads when the base is aligned (all callers pass tensor bases)
-    long long n4 = (reinterpret_cast<uintptr_t>(a) & 15) == 0 ? n / 4 : 0;
+    const long long n4 = (reinterpret_cast<uintptr_t>(a) & 15) == 0 ? n / 4 : 0;
     const float4 *a4 = reinterpret_cast<const float4 *>(a);
-    for (long long j = i; j < n4; j += stride) {
-        float4 v = a4[j];
-        // NaN lanes are skipped (compare-false keeps the running value)
+    // NaN lanes are skipped (compare-false keeps the running value)
+    auto take = [&](const float4 &v) {
         lo = v.x < lo ? v.x : lo; hi = v.x > hi ? v.x : hi;
         lo = v.y < lo ? v.y : lo; hi = v.y > hi ? v.y : hi;
         lo = v.z < lo ? v.z : lo; hi = v.z > hi ? v.z : hi;
         lo = v.w < lo ? v.w : lo; hi = v.w > hi ? v.w : hi;
+    };
+    // DQ_MMU loads in flight a pass: the partials allow no more than 256
+    // workgroups, so a large A is many passes (2048 x 2048: 5.5 -> 4.0 us)
+    long long j = i;
+    for (; j + (DQ_MMU - 1) * stride < n4; j += DQ_MMU * stride) {
+        float4 v[DQ_MMU];
+#pragma unroll
+        for (int u = 0; u < DQ_MMU; u++) v[u] = a4[j + u * stride];
+#pragma unroll
+        for (int u = 0; u < DQ_MMU; u++) take(v[u]);
     }
-    for (long long j = n4 * 4 + i; j < n; j += stride) {
+    for (; j < n4; j += stride) take(a4[j]);
+    for (j = n4 * 4 + i; j < n; j += stride) {
         float v = a[j];
         lo = v < lo ? v : lo;
         hi = v > hi ? v : hi;
@@ -183,122 +198,55 @@ __device__ __forceinline__ int quantize_one(float x, float inv, float zpf) {
     return (int)q;
 }
 
-// One wave per row of A (padded rows write zeros): each lane quantizes 4
-// consecutive k per step (one 16-byte load, one 4-byte store into the lane's
-// operand slot), and the row sum of a'' and the NaN flag are wave reductions,
-// so the kernel needs no atomics and no zeroed scratch.
+// Four consecutive k of one row.
 struct Quad {
     float v[4];
 };
 
-// x[kk .. kk+3] of one row (zeros past k or for padding rows).
-__device__ __forceinline__ Quad load_quad(const float *__restrict__ src, int kk, int k, bool live, bool vec) {
-    Quad q = {{0.f, 0.f, 0.f, 0.f}};
-    if (live && kk < k) {
-        if (vec) {
-            float4 v = *reinterpret_cast<const float4 *>(src + kk);
-            q.v[0] = v.x; q.v[1] = v.y; q.v[2] = v.z; q.v[3] = v.w;
-        } else {
-#pragma unroll
-            for (int b = 0; b < 4; b++) q.v[b] = kk + b < k ? src[kk + b] : 0.f;
-        }
-    }
-    return q;
-}
+// MatMulInteger's activations: u8 (a - 128) or s8 (a) into the s8 a'' of the
+// MFMA layout.  A wave takes DQ_MF fragments (32 rows x 32 k) of one row tile:
+// lane l loads 16 consecutive bytes of row l & 31, k half l >> 5 -- with one
+// 16-byte load where every row is 16-byte aligned -- and stores them at l * 16.
+// Block 0 publishes alpha = (u8 ? 128 : 0) - a_zp so that a - a_zp = a'' +
+// alpha; no row is NaN.
+constexpr int DQ_MF = 4;
 
-constexpr int DQ_QPRE = 4;  // row chunks of 256 loaded before the parameter reduction
-
-__global__ __launch_bounds__(DQ_THREADS) void dqmm_quantize_kernel(const float *__restrict__ a, int m, int k,
-                                                                    DqScratch *__restrict__ sc, int nparts,
-                                                                    int *__restrict__ qparams,
-                                                                    int *__restrict__ rowsum,
-                                                                    int8_t *__restrict__ apk) {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * (DQ_THREADS / 64) + (threadIdx.x >> 6);
-    const int kpad = pad32(k), mpad = pad32(m);
-    const bool live = row < m;
-    const float *src = a + (long long)(live ? row : 0) * k;
-    const bool vec = (k & 3) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
-    // The first chunks of the row are in flight while the block reduces the
-    // min/max partials.
-    Quad pre[DQ_QPRE];
-#pragma unroll
-    for (int c = 0; c < DQ_QPRE; c++) pre[c] = load_quad(src, 4 * lane + 256 * c, k, live, vec);
-    float inv;
-    int zp;
-    dq_params(sc, nparts, qparams, blockIdx.x == 0, inv, zp);
-    if (row >= mpad) return;
-    const float zpf = (float)zp;
-    int *dst = reinterpret_cast<int *>(apk) + (long long)(row >> 5) * (kpad / 32) * 256 + (row & 31) * 4;
-    int sum = 0;
-    bool nan = false;
-    auto emit = [&](const Quad &x, int kk) {
-        unsigned packed = 0;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            int v = 0;  // padding rows/columns carry a'' = 0
-            if (live && kk + b < k) {
-                float p = x.v[b] * inv;
-                nan |= !(p == p);
-                v = quantize_one(x.v[b], inv, zpf) - 128;
-                sum += v;
-            }
-            packed |= (unsigned)(v & 0xff) << (8 * b);
-        }
-        // fragment (row/32, kk/32); lane slot (row & 31) + 32 * ((kk >> 4) & 1); byte kk & 15
-        dst[(kk >> 5) * 256 + ((kk >> 4) & 1) * 128 + ((kk & 15) >> 2)] = (int)packed;
-    };
-#pragma unroll
-    for (int c = 0; c < DQ_QPRE; c++) {
-        const int kk = 4 * lane + 256 * c;
-        if (kk < kpad) emit(pre[c], kk);
-    }
-    for (int kk = 4 * lane + 256 * DQ_QPRE; kk < kpad; kk += 256) emit(load_quad(src, kk, k, live, vec), kk);
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-    const bool any_nan = __any(nan);
-    if (lane == 0) {
-        rowsum[row] = sum;
-        rowsum[mpad + row] = any_nan ? 1 : 0;
-    }
-}
-
-// MatMulInteger's activations: one wave per row turns u8 (a - 128) or s8 (a)
-// into the s8 a'' of the MFMA layout and sums each row; block 0 publishes
-// alpha = (u8 ? 128 : 0) - a_zp so that a - a_zp = a'' + alpha.
 __global__ __launch_bounds__(DQ_THREADS) void mmi_pack_a_kernel(const uint8_t *__restrict__ a, int m, int k,
                                                                  int a_signed, int a_zp, DqScratch *__restrict__ sc,
-                                                                 int *__restrict__ rowsum, int8_t *__restrict__ apk) {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * (DQ_THREADS / 64) + (threadIdx.x >> 6);
-    const int kpad = pad32(k), mpad = pad32(m);
+                                                                 int *__restrict__ rownan, int8_t *__restrict__ apk) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ks = pad32(k) / 32, nch = (ks + DQ_MF - 1) / DQ_MF;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         sc->alpha = (a_signed ? 0 : 128) - a_zp;
         sc->scale = 1.0f;
         sc->zp = a_zp;
     }
-    if (row >= mpad) return;
+    const int w = blockIdx.x * (DQ_THREADS / 64) + wave;
+    const int mt = w / nch, s0 = w % nch * DQ_MF;
+    if (mt * 32 >= m) return;
+    const int row = mt * 32 + (lane & 31);
     const bool live = row < m;
+    if (s0 == 0 && lane < 32) rownan[row] = 0;
     const uint8_t *src = a + (long long)(live ? row : 0) * k;
-    int *dst = reinterpret_cast<int *>(apk) + (long long)(row >> 5) * (kpad / 32) * 256 + (row & 31) * 4;
-    int sum = 0;
-    for (int kk = 4 * lane; kk < kpad; kk += 256) {
-        unsigned packed = 0;
+    const bool vec = (k & 15) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+    const unsigned flip = a_signed ? 0u : 0x80808080u;  // u8 - 128, byte by byte
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            int v = 0;  // padding rows/columns carry a'' = 0
-            if (live && kk + b < k) {
-                const int raw = src[kk + b];
-                v = a_signed ? (int)(int8_t)raw : raw - 128;
-                sum += v;
+    for (int f = 0; f < DQ_MF; f++) {
+        const int s = s0 + f, kk = s * 32 + 16 * (lane >> 5);
+        i32x4 v = {};  // padding rows and columns carry a'' = 0
+        if (live && vec) {
+            if (kk < k) {
+                v = *reinterpret_cast<const i32x4 *>(src + kk);
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] ^= (int)flip;
             }
-            packed |= (unsigned)(v & 0xff) << (8 * b);
+        } else if (live) {
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+                if (kk + e < k)
+                    v[e >> 2] |= (int)(((unsigned)src[kk + e] ^ (flip & 0xffu)) << (8 * (e & 3)));
         }
-        dst[(kk >> 5) * 256 + ((kk >> 4) & 1) * 128 + ((kk & 15) >> 2)] = (int)packed;
-    }
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-    if (lane == 0) {
-        rowsum[row] = sum;
-        rowsum[mpad + row] = 0;
+        if (s < ks) *reinterpret_cast<i32x4 *>(apk + (((long long)mt * ks + s) * 64 + lane) * 16) = v;
     }
 }
 
@@ -346,96 +294,173 @@ __global__ void dqmm_pack_kernel(int k, int n, const void *__restrict__ w, int w
     off[j] = j < n ? o : 0;
 }
 
-// Wave tile 32 x 32, 4 waves per block as 2 x 2 -> 64 x 64 outputs per block.
-__global__ __launch_bounds__(256) void dqmm_gemm_kernel(int m, int k, int n, const int8_t *__restrict__ apk,
-                                                        const int8_t *__restrict__ wpk,
-                                                        const int *__restrict__ colsum, const int *__restrict__ off,
-                                                        const int *__restrict__ rowsum,
-                                                        const DqScratch *__restrict__ sc,
-                                                        const float *__restrict__ wscale, int n_wscale,
-                                                        const float *__restrict__ bias, float *__restrict__ out,
-                                                        int *__restrict__ acc_out) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int mt = blockIdx.y * 2 + (wave >> 1);
-    const int nt = blockIdx.x * 2 + (wave & 1);
-    const int kpad = pad32(k), ks = kpad / 32;
-    if (mt * 32 >= pad32(m) || nt * 32 >= pad32(n)) return;
-    const i32x4 *A = reinterpret_cast<const i32x4 *>(apk) + (long long)mt * ks * 64 + lane;
-    const i32x4 *B = reinterpret_cast<const i32x4 *>(wpk) + (long long)nt * ks * 64 + lane;
-    // Epilogue operands are loaded before the k loop so their latency overlaps it.
-    // The lane's 16 rows are 4 runs of 4 consecutive rows: their row sums and
-    // NaN flags are 8 int4 loads (rows are padded to mpad, columns to npad).
-    const int j = nt * 32 + (lane & 31);
-    const int mpad = pad32(m);
-    int4 rs[4], rn[4];
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const int i0 = mt * 32 + 8 * g + 4 * (lane >> 5);
-        rs[g] = *reinterpret_cast<const int4 *>(rowsum + i0);
-        rn[g] = *reinterpret_cast<const int4 *>(rowsum + mpad + i0);
-    }
-    // two's-complement wrap-around below is exact as long as the final sum fits in int32
-    const unsigned offj = (unsigned)off[j];
-    const int csum = colsum[j];
-    const float ws = (wscale && j < n) ? (n_wscale == 1 ? wscale[0] : wscale[j]) : 0.0f;
-    const float bj = (bias && j < n) ? bias[j] : 0.0f;
-    const int aalpha = sc->alpha;
-    const float ascale = sc->scale;
-    // k in chunks of DQ_KC steps: the next chunk's 2*DQ_KC loads are in flight
-    // while the current chunk's MFMAs run.
-    i32x16 acc = {};
-    i32x4 a[DQ_KC], b[DQ_KC];
-    const int full = ks / DQ_KC;
-    if (full > 0) {
-#pragma unroll
-        for (int t = 0; t < DQ_KC; t++) {
-            a[t] = A[t * 64];
-            b[t] = B[t * 64];
-        }
-    }
-    for (int c = 0; c < full; c++) {
-        i32x4 na[DQ_KC], nb[DQ_KC];
-        const bool more = c + 1 < full;
-        if (more) {
-#pragma unroll
-            for (int t = 0; t < DQ_KC; t++) {
-                na[t] = A[((c + 1) * DQ_KC + t) * 64];
-                nb[t] = B[((c + 1) * DQ_KC + t) * 64];
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < DQ_KC; t++) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[t], b[t], acc, 0, 0, 0);
-        if (more) {
-#pragma unroll
-            for (int t = 0; t < DQ_KC; t++) {
-                a[t] = na[t];
-                b[t] = nb[t];
-            }
-        }
-    }
-    for (int s = full * DQ_KC; s < ks; s++)
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[s * 64], B[s * 64], acc, 0, 0, 0);
+// What the epilogue needs of output column j: loaded without a condition (a
+// lane past the last column reads the last one's and stores nothing), so that
+// nothing waits before the operand loads that follow.
+struct ColOperands {
+    int off, csum;
+    float ws, bias;
+};
+__device__ __forceinline__ ColOperands load_column(int j, int n, const int *__restrict__ colsum,
+                                                   const int *__restrict__ off, const float *__restrict__ wscale,
+                                                   int n_wscale, const float *__restrict__ bias) {
+    const int jc = j < n ? j : n - 1;
+    ColOperands c;
+    c.off = off[jc];
+    c.csum = colsum[jc];
+    c.ws = wscale ? wscale[n_wscale == 1 ? 0 : jc] : 0.0f;
+    c.bias = bias ? bias[jc] : 0.0f;
+    return c;
+}
 
-    if (j >= n) return;
-    const unsigned alpha = (unsigned)aalpha;
-    const unsigned colterm = alpha * (unsigned)csum + (unsigned)k * alpha * offj;
-    const float comb = ascale * ws;  // CombinedScale, QuantizedMatMulOps.cs:203-221
+// The int8 GEMM over packed operands.  A workgroup owns 32 TM rows x 128
+// columns; each of its four waves one 32-column tile and all TM row tiles, on
+// v_mfma_i32_32x32x32_i8.
+//
+// Fragments are 1 KB (one 32-row or 32-column tile x 32 k, already in the
+// MFMA's lane order).  A wave's W fragments are its own, so they come straight
+// into registers; the A fragments, which all four waves read, go through LDS,
+// four k-steps a stage: wave w loads k-step w of every row tile, one barrier a
+// stage, two buffers, lane l at l * 16 (no bank conflicts).  SETS stages
+// are in flight in registers.
+//
+// Each tile has its own buffer descriptor of exactly its k-steps (none for a
+// tile past the last): loads past it return zeros and fetch nothing, which
+// ends the prefetch and pads the last stage without a branch.  Row sums of a''
+// come from the staged registers (v_dot4).
+//
+// Bound by LDS and L1 traffic and, at the ends, the first loads and the output
+// stores: 1028 x 1280 x 5120 takes 18.5 us here (13.5 G int-ops, 727 TOP/s; 4
+// us of it stores, 6 the first loads and the epilogue), 512 x 512 x 2048 4.8.
+constexpr int DQG_KS = 4;
+enum { DQG_FLOAT = 1, DQG_ACC = 2 };  // which outputs a launch writes
+
+template <int TM, int SETS, int OUT>
+__global__ __launch_bounds__(256, 2) void dqmm_gemm_kernel(int m, int k, int n, const int8_t *__restrict__ apk,
+                                                           const int8_t *__restrict__ wpk,
+                                                           const int *__restrict__ colsum,
+                                                           const int *__restrict__ off,
+                                                           const int *__restrict__ rownan,
+                                                           const DqScratch *__restrict__ sc,
+                                                           const float *__restrict__ wscale, int n_wscale,
+                                                           const float *__restrict__ bias, float *__restrict__ out,
+                                                           int *__restrict__ acc_out) {
+    static_assert(DQG_KS == 4 && SETS % 2 == 0, "a wave loads one k-step of a stage; buffers alternate");
+    static_assert(32 * TM <= 256, "one row sum a thread");
+    __shared__ __align__(16) i32x4 frag[2][TM * DQG_KS * 64];
+    __shared__ __align__(16) int lds_rs[32 * TM], lds_rn[32 * TM];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = pad32(k) / 32, nmt = pad32(m) / 32, nnt = pad32(n) / 32, mpad = pad32(m);
+    // XCD-banded ids, rows first: an XCD's workgroups share a band of W's
+    // columns and all of A's rows
+    const int nmb = (nmt + TM - 1) / TM;
+    const int id = xcd_band(blockIdx.x, gridDim.x);
+    const int mt0 = (id % nmb) * TM, nt = (id / nmb) * 4 + wave;
+
+    struct Set {
+        i32x4 a[TM], b[DQG_KS];
+    };
+    auto load_tile = [&](const int8_t *base, int tile, int ntiles, int voff) {
+        const bool live = tile < ntiles;
+        __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(base + (live ? (long long)tile * ks * 1024 : 0)), (short)0, live ? ks * 1024 : 0, 0x00020000);
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, 0, 0);
+        return i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+    };
+    auto load = [&](Set &r, int st) {
+        const int voff = lane * 16 + st * DQG_KS * 1024;
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int i = mt * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int4 s4 = rs[r >> 2], n4 = rn[r >> 2];
-        const int rsum = (r & 3) == 0 ? s4.x : (r & 3) == 1 ? s4.y : (r & 3) == 2 ? s4.z : s4.w;
-        const int rnan = (r & 3) == 0 ? n4.x : (r & 3) == 1 ? n4.y : (r & 3) == 2 ? n4.z : n4.w;
-        if (i < m) {
-            int v = (int)((unsigned)acc[r] + offj * (unsigned)rsum + colterm);
-            if (acc_out) acc_out[(long long)i * n + j] = v;
-            if (out) {
-                float o = __builtin_fmaf((float)v, comb, bj);
-                if (rnan) o = __builtin_nanf("");
-                out[(long long)i * n + j] = o;
-            }
+        for (int t = 0; t < TM; t++) r.a[t] = load_tile(apk, mt0 + t, nmt, voff + wave * 1024);
+#pragma unroll
+        for (int kk = 0; kk < DQG_KS; kk++) r.b[kk] = load_tile(wpk, nt, nnt, voff + kk * 1024);
+    };
+    auto stage = [&](const Set &r, int buf) {
+#pragma unroll
+        for (int t = 0; t < TM; t++) frag[buf][(t * DQG_KS + wave) * 64 + lane] = r.a[t];
+    };
+    const int nst = (ks + DQG_KS - 1) / DQG_KS;
+    Set r[SETS];
+#pragma unroll
+    for (int u = 0; u < SETS; u++) load(r[u], u);
+    // the epilogue's operands: NaN flags (and, after the loop, the row sums)
+    // through LDS, columns in registers
+    if (tid < 32 * TM) {
+        lds_rs[tid] = 0;
+        lds_rn[tid] = rownan[mt0 * 32 + tid < mpad ? mt0 * 32 + tid : 0];
+    }
+    const int j = nt * 32 + (lane & 31);
+    const bool jlive = j < n;
+    const ColOperands col = load_column(j, n, colsum, off, wscale, n_wscale, bias);
+    const unsigned alpha = (unsigned)sc->alpha;
+    const float ascale = sc->scale;
+
+    i32x16 acc[TM] = {};
+    int rsum[TM] = {};  // sum of a'' over this wave's k-steps of row lane & 31 (and k half lane >> 5)
+    auto add_rows = [&](const Set &r) {
+#pragma unroll
+        for (int t = 0; t < TM; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) rsum[t] = __builtin_amdgcn_sdot4(r.a[t][e], 0x01010101, rsum[t], false);
+    };
+    stage(r[0], 0);
+    add_rows(r[0]);
+    __syncthreads();
+    for (int st = 0; st < nst; st += SETS) {
+#pragma unroll
+        for (int u = 0; u < SETS; u++) {
+            // LDS buffer u & 1 holds stage st + u's A, r[u] its W; the other
+            // sets the stages after it; stages past the last are zeros
+            const i32x4 *fa = frag[u & 1] + lane;
+#pragma unroll
+            for (int kk = 0; kk < DQG_KS; kk++)
+#pragma unroll
+                for (int t = 0; t < TM; t++)
+                    acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[(t * DQG_KS + kk) * 64], r[u].b[kk], acc[t], 0,
+                                                                   0, 0);
+            load(r[u], st + u + SETS);
+            stage(r[(u + 1) % SETS], (u + 1) & 1);
+            add_rows(r[(u + 1) % SETS]);
+            __syncthreads();
         }
     }
+#pragma unroll
+    for (int t = 0; t < TM; t++) atomicAdd(lds_rs + t * 32 + (lane & 31), rsum[t]);
+    __syncthreads();
+    if (!jlive) return;
+    // Epilogue.  two's-complement wrap-around is exact as long as the final sum
+    // fits in int32.  A zero point and a row sum fit 24 bits (|sum a''| <=
+    // 128 * 33025), so the row term is one full-rate mad.
+    const int half = lane >> 5;
+    const int offj = col.off;
+    const float bj = col.bias;
+    const int colterm = (int)(alpha * (unsigned)col.csum + (unsigned)k * alpha * (unsigned)offj);
+    const float comb = ascale * col.ws;  // CombinedScale, QuantizedMatMulOps.cs:203-221
+    auto epilogue = [&](auto full) {  // full: every row is inside the matrix
+#pragma unroll
+        for (int t = 0; t < TM; t++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int il = t * 32 + 8 * q + 4 * half;
+                const int4 s4 = *reinterpret_cast<const int4 *>(lds_rs + il);
+                const int4 n4 = *reinterpret_cast<const int4 *>(lds_rn + il);
+                const long long at = (long long)(mt0 * 32 + il) * n + j;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int rs = e == 0 ? s4.x : e == 1 ? s4.y : e == 2 ? s4.z : s4.w;
+                    const int rnan = e == 0 ? n4.x : e == 1 ? n4.y : e == 2 ? n4.z : n4.w;
+                    if (full || mt0 * 32 + il + e < m) {
+                        const int v = (int)((unsigned)acc[t][4 * q + e] + (unsigned)(__mul24(offj, rs) + colterm));
+                        if constexpr (OUT & DQG_ACC) acc_out[at + (long long)e * n] = v;
+                        if constexpr (OUT & DQG_FLOAT) {
+                            const float o = __builtin_fmaf((float)v, comb, bj);
+                            out[at + (long long)e * n] = rnan ? __builtin_nanf("") : o;
+                        }
+                    }
+                }
+            }
+    };
+    if ((mt0 + TM) * 32 <= m) epilogue(std::true_type{});
+    else epilogue(std::false_type{});
 }
 
 // Quantize + GEMM in one launch, after dqmm_minmax_kernel.  A workgroup owns
@@ -488,6 +513,82 @@ __device__ __forceinline__ unsigned quantize4(const Quad &x, float inv, float zp
     return packed;
 }
 
+// The quantize launch: a wave takes DQ_QF fragments (32 rows x 32 k) of one row
+// tile.  Lane l loads four consecutive k of row l / 8 + 8 i -- a row's 8 lanes
+// one whole 128-byte line -- all before the parameter reduction, and stores the
+// packed four bytes into the fragment, 128 contiguous bytes per eight rows.
+// A row with a NaN raises its flag, which the min/max launch cleared; the
+// GEMM sums the rows itself.
+constexpr int DQ_QF = 2;
+
+__global__ __launch_bounds__(DQ_THREADS) void dqmm_quantize_kernel(const float *__restrict__ a, int m, int k,
+                                                                    DqScratch *__restrict__ sc, int nparts,
+                                                                    int *__restrict__ qparams,
+                                                                    int *__restrict__ rownan,
+                                                                    int8_t *__restrict__ apk) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ks = pad32(k) / 32;
+    const int nch = (ks + DQ_QF - 1) / DQ_QF;
+    const int w = blockIdx.x * (DQ_THREADS / 64) + wave;
+    const int mt = w / nch, s0 = w % nch * DQ_QF;
+    const bool any = mt * 32 < m;
+    const int r8 = lane >> 3, c8 = lane & 7;
+    // Unconditional loads: a descriptor of the row tile's rows, an offset past
+    // it for rows and columns that do not exist (zeros, nothing fetched).  A
+    // quad that crosses k reads into the next row, masked below; 4-byte
+    // alignment is all a buffer load needs.
+    const int rows = any ? (m - mt * 32 < 32 ? m - mt * 32 : 32) : 0;
+    __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)(a + (any ? (long long)mt * 32 * k : 0)),
+                                                                  (short)0, rows * k * 4, 0x00020000);
+    Quad x[DQ_QF][4];
+#pragma unroll
+    for (int f = 0; f < DQ_QF; f++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int kk = (s0 + f) * 32 + 4 * c8;
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(ra, kk < k ? ((8 * i + r8) * k + kk) * 4 : -1, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[f][i].v[e] = __uint_as_float(v[e]);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    float inv;
+    int zp;
+    dq_params(sc, nparts, qparams, blockIdx.x == 0, inv, zp);
+    if (!any) return;
+    const float zpf = (float)zp;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int row = mt * 32 + 8 * i + r8;
+        int sum = 0;
+        bool nan = false;
+#pragma unroll
+        for (int f = 0; f < DQ_QF; f++) {
+            const int s = s0 + f, kk = s * 32 + 4 * c8;
+            unsigned lm = 0;  // padding rows and columns carry a'' = 0
+#pragma unroll
+            for (int e = 0; e < 4; e++) lm |= (row < m && kk + e < k) ? (1u << e) : 0u;
+            // fragment (mt, s); lane slot (row & 31) + 32 * (c8 >> 2); byte 4 (c8 & 3)
+            const unsigned q = quantize4(x[f][i], inv, zpf, lm, sum, nan);
+            if (s < ks)
+                reinterpret_cast<unsigned *>(
+                    apk)[((long long)mt * ks + s) * 256 + (8 * i + r8 + 32 * (c8 >> 2)) * 4 + (c8 & 3)] = q;
+        }
+        if (nan) atomicOr(rownan + row, 1);
+    }
+}
+
+// The same with every element live and the sum left to the caller.
+__device__ __forceinline__ unsigned quantize4(const Quad &x, float inv, float zpf, bool &nan) {
+    unsigned packed = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float p = x.v[e] * inv;
+        nan |= !(p == p);
+        packed = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_rintf(p) + zpf, e, packed);
+    }
+    return packed ^ 0x80808080u;  // q -> q - 128, byte by byte
+}
+
 // FULL: m % 32 == 0, n % 128 == 0, k % 512 == 0 and A 16-byte aligned, so
 // every row, column and k-step is live and no load or store needs a check.
 // The host picks it whenever it applies; the kernel then has no divergent
@@ -522,9 +623,6 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     const int row = mt * 32 + r;
     const bool live = FULL || row < m;
     const float *src = a + (long long)(live ? row : 0) * k;
-    const bool vec = FULL || ((k & 3) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0);
-    // all 32 rows live and 16-byte loads: passes inside k need no per-element checks
-    const bool rows_full = FULL || (vec && mt * 32 + 32 <= m);
     const int npass = (ks + DQF_KS - 1) / DQF_KS;
     const i32x4 *B = reinterpret_cast<const i32x4 *>(wpk) + (long long)(col_live ? nt : 0) * ks * 64 + lane;
 
@@ -535,31 +633,43 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     // the epilogue's column operands, loaded now so their latency hides under the pass
     const int j = nt * 32 + (lane & 31);
     const bool jlive = col_live && (FULL || j < n);
-    const int offj_raw = jlive ? off[j] : 0;
-    const int csum = jlive ? colsum[j] : 0;
-    const float ws = jlive ? (n_wscale == 1 ? wscale[0] : wscale[j]) : 0.0f;
-    const float bj = (jlive && bias) ? bias[j] : 0.0f;
+    const ColOperands col = load_column(j, n, colsum, off, wscale, n_wscale, bias);
 
     Quad x[DQF_KS];
     i32x4 b[DQF_KS];
+    // Without FULL the loads go through buffer descriptors (of the row tile's
+    // rows, of the column tile's k-steps): rows, columns and k-steps that do
+    // not exist return zeros and fetch nothing, so every load is unconditional
+    // and in flight at once; a quad that crosses k reads into the next row and
+    // is masked when quantized.  (Guarded loads merged their registers by
+    // copies that waited for each other: 70 x 96 x 300 9.5 us.)
+    const int rows = m - mt * 32 < 32 ? m - mt * 32 : 32;
+    __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)(a + (long long)mt * 32 * k), (short)0,
+                                                                  rows * k * 4, 0x00020000);
+    __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(wpk + (col_live ? (long long)nt * ks * 1024 : 0)), (short)0, col_live ? ks * 1024 : 0, 0x00020000);
     auto load_pass = [&](int s0) {
-        if (FULL || (rows_full && (s0 + DQF_KS) * 32 <= k)) {
+        if constexpr (FULL) {
 #pragma unroll
             for (int i = 0; i < DQF_KS; i++) {
                 const float4 v = *reinterpret_cast<const float4 *>(src + (s0 + i) * 32 + 4 * c8);
                 x[i].v[0] = v.x; x[i].v[1] = v.y; x[i].v[2] = v.z; x[i].v[3] = v.w;
             }
-        } else {
-#pragma unroll
-            for (int i = 0; i < DQF_KS; i++) x[i] = load_quad(src, (s0 + i) * 32 + 4 * c8, k, live, vec);
-        }
-        if (FULL) {
 #pragma unroll
             for (int t = 0; t < DQF_KS; t++) b[t] = B[(s0 + t) * 64];
-        } else if (col_live) {
+        } else {
 #pragma unroll
-            for (int t = 0; t < DQF_KS; t++)
-                if (s0 + t < ks) b[t] = B[(s0 + t) * 64];
+            for (int i = 0; i < DQF_KS; i++) {
+                const int kk = (s0 + i) * 32 + 4 * c8;
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(ra, kk < k ? (r * k + kk) * 4 : -1, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[i].v[e] = __uint_as_float(v[e]);
+            }
+#pragma unroll
+            for (int t = 0; t < DQF_KS; t++) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + (s0 + t) * 1024, 0, 0);
+                b[t] = i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+            }
         }
     };
     load_pass(0);
@@ -581,14 +691,24 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     int *dst = lds_a + (r + 32 * (c8 >> 2)) * 4 + (c8 & 3);
     for (int ps = 0; ps < npass; ps++) {
         const int s0 = ps * DQF_KS;
-        if (FULL || (rows_full && (s0 + DQF_KS) * 32 <= k)) {
+        if constexpr (FULL) {
 #pragma unroll
             for (int i = 0; i < DQF_KS; i++) dst[i * 256] = (int)quantize4(x[i], inv, zpf, 0xfu, sum, nan);
         } else {
+            // k % 4 == 0: a quad is all inside its row or not there at all (its
+            // loads then gave zeros: no NaN), so one select masks it
+            if ((k & 3) == 0) {
 #pragma unroll
-            for (int i = 0; i < DQF_KS; i++) {
-                const int kk = (s0 + i) * 32 + 4 * c8;
-                if (kk < kpad) {
+                for (int i = 0; i < DQF_KS; i++) {
+                    const unsigned q = quantize4(x[i], inv, zpf, nan);
+                    const int v = live && (s0 + i) * 32 + 4 * c8 < k ? (int)q : 0;
+                    sum = __builtin_amdgcn_sdot4(v, 0x01010101, sum, false);
+                    dst[i * 256] = v;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < DQF_KS; i++) {
+                    const int kk = (s0 + i) * 32 + 4 * c8;
                     unsigned lm = 0;
 #pragma unroll
                     for (int e = 0; e < 4; e++) lm |= (live && kk + e < k) ? (1u << e) : 0u;
@@ -597,9 +717,9 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
             }
         }
         __syncthreads();
-        if (col_live) {
+        {
             const int *srcl = lds_a + lane * 4;
-            if (FULL || s0 + DQF_KS <= ks) {
+            if (FULL || s0 + DQF_KS <= ks) {  // k-steps past the last are zeros
                 i32x4 av[DQF_KS];
 #pragma unroll
                 for (int t = 0; t < DQF_KS; t++) av[t] = *reinterpret_cast<const i32x4 *>(srcl + t * 256);
@@ -641,10 +761,11 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     }
     __syncthreads();
     if (!jlive) return;
-    const unsigned offj = (unsigned)offj_raw;
+    const unsigned offj = (unsigned)col.off;
+    const float bj = col.bias;
     const unsigned alpha = (unsigned)(128 - zp);
-    const unsigned colterm = alpha * (unsigned)csum + (unsigned)k * alpha * offj;
-    const float comb = scale * ws;  // CombinedScale, QuantizedMatMulOps.cs:203-221
+    const unsigned colterm = alpha * (unsigned)col.csum + (unsigned)k * alpha * offj;
+    const float comb = scale * col.ws;  // CombinedScale, QuantizedMatMulOps.cs:203-221
     if constexpr (FULL) {
         // Float output only, 16-byte aligned: the wave's 32 x 32 tile goes
         // through its own 4 KB of lds_a (every wave's A reads ended before
@@ -865,13 +986,166 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused16_kernel(
     epilogue(3);
 }
 
-static osh_status run_minmax(const float *a, long long count, DqScratch *sc, int *nparts, hipStream_t st) {
+// Quantize + GEMM for at most RT <= 16 rows (a token, a few beams), after
+// dqmm_minmax_kernel.  A 32-row tile would leave most threads without a row to
+// quantize and a 128-column workgroup most CUs without work (3 x 1912 x 168 ran
+// on two workgroups, 28 us), so here a workgroup owns 32 columns and its four
+// waves split K, k-step s to wave s % 4; the sums meet in LDS, exact in int32.
+// 256 / RT threads quantize each row, DQS_KS k-steps a pass; every wave's W
+// fragments of two passes (K = 2048) are in flight before the parameter
+// reduction.  Rows of the A tile past m are whatever LDS held: they reach only
+// output rows that do not exist; k-steps past the last meet zero W.
+constexpr int DQS_KS = 32;  // k-steps a pass
+constexpr int DQS_WS = DQS_KS / 4;
+
+template <int RT>
+__global__ __launch_bounds__(256) void dqmm_skinny_kernel(
+    int m, int k, int n, const float *a, DqScratch *__restrict__ sc, int nparts, int *__restrict__ qparams,
+    const int8_t *wpk, const int *__restrict__ colsum, const int *__restrict__ off,
+    const float *__restrict__ wscale, int n_wscale, const float *__restrict__ bias, float *__restrict__ out,
+    int *__restrict__ acc_out) {
+    static_assert(RT <= 16, "two row quads of the accumulator");
+    constexpr int TPR = 256 / RT;  // threads a row
+    __shared__ __attribute__((aligned(16))) int lds_a[DQS_KS * 256];  // [kstep][64 lanes][16 bytes]
+    __shared__ int lds_acc[4][8][64];
+    __shared__ int lds_rs[RT], lds_rn[RT];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = pad32(k) / 32, nt = blockIdx.x;
+    const int r = tid / TPR, c = tid % TPR;
+    const int pidx = tid < nparts ? tid : 0;
+    const float pmin = sc->partial_min[pidx], pmax = sc->partial_max[pidx];
+    const int oc = tid & 31, j = nt * 32 + oc;  // the output column this thread ends with
+    const ColOperands col = load_column(j, n, colsum, off, wscale, n_wscale, bias);
+    __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)a, (short)0, m * k * 4, 0x00020000);
+    __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)(wpk + (long long)nt * ks * 1024), (short)0,
+                                                                  ks * 1024, 0x00020000);
+    Quad x[RT];  // quad i of this thread: k = 32 s0 + 4 (c + TPR i)
+    auto load_a = [&](int s0) {
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+            const int kk = s0 * 32 + 4 * (c + TPR * i);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(ra, kk < k ? (r * k + kk) * 4 : -1, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[i].v[e] = __uint_as_float(v[e]);
+        }
+    };
+    i32x4 b[2][DQS_WS];
+    auto load_b = [&](i32x4 (&bb)[DQS_WS], int s0) {
+#pragma unroll
+        for (int t = 0; t < DQS_WS; t++) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + (s0 + 4 * t + wave) * 1024, 0, 0);
+            bb[t] = i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+        }
+    };
+    load_a(0);
+    load_b(b[0], 0);
+    load_b(b[1], DQS_KS);
+    if (tid < RT) lds_rs[tid] = lds_rn[tid] = 0;
+    __builtin_amdgcn_sched_barrier(0);
+    float inv, scale;
+    int zp;
+    dq_finish(sc, __builtin_fminf(0.f, pmin), __builtin_fmaxf(0.f, pmax), qparams, blockIdx.x == 0, inv, zp,
+              &scale);
+    const float zpf = (float)zp;
+    int sum = 0;
+    bool nan = false;
+    i32x16 acc0 = {}, acc1 = {};
+    auto pass = [&](i32x4 (&bb)[DQS_WS], int s0) {
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+            const int kl = 4 * (c + TPR * i), kk = s0 * 32 + kl;
+            unsigned lm = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) lm |= (r < m && kk + e < k) ? (1u << e) : 0u;
+            lds_a[(kl >> 5) * 256 + (r + 32 * ((kl >> 4) & 1)) * 4 + ((kl & 15) >> 2)] =
+                (int)quantize4(x[i], inv, zpf, lm, sum, nan);
+        }
+        __syncthreads();
+        const int *src = lds_a + lane * 4;
+#pragma unroll
+        for (int t = 0; t < DQS_WS; t += 2) {
+            acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                *reinterpret_cast<const i32x4 *>(src + (4 * t + wave) * 256), bb[t], acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                *reinterpret_cast<const i32x4 *>(src + (4 * t + 4 + wave) * 256), bb[t + 1], acc1, 0, 0, 0);
+        }
+        if (s0 + DQS_KS < ks) {
+            load_a(s0 + DQS_KS);
+            load_b(bb, s0 + 2 * DQS_KS);
+            __syncthreads();  // every wave has read the pass before it is rewritten
+        }
+    };
+    for (int s0 = 0; s0 < ks; s0 += 2 * DQS_KS) {
+        pass(b[0], s0);
+        if (s0 + DQS_KS < ks) pass(b[1], s0 + DQS_KS);
+    }
+    // a row's threads: whole waves, or consecutive lanes of one
+#pragma unroll
+    for (int o = 1; o < (TPR < 64 ? TPR : 64); o <<= 1) {
+        sum += __shfl_xor(sum, o);
+        const int other = __shfl_xor(nan ? 1 : 0, o);
+        nan = nan || other != 0;
+    }
+    if ((tid & ((TPR < 64 ? TPR : 64) - 1)) == 0) {
+        atomicAdd(lds_rs + r, sum);
+        if (nan) lds_rn[r] = 1;
+    }
+#pragma unroll
+    for (int v = 0; v < 8; v++) lds_acc[wave][v][lane] = acc0[v] + acc1[v];
+    __syncthreads();
+    if (j >= n) return;
+    const unsigned alpha = (unsigned)(128 - zp), offj = (unsigned)col.off;
+    const unsigned colterm = alpha * (unsigned)col.csum + (unsigned)k * alpha * offj;
+    const float comb = scale * col.ws;  // CombinedScale, QuantizedMatMulOps.cs:203-221
+    for (int row = tid >> 5; row < m; row += 8) {
+        // the accumulator's row 8 q + 4 half + e: register 4 q + e of lane column + 32 half
+        const int reg = 4 * (row >> 3) + (row & 3), l = oc + 32 * ((row >> 2) & 1);
+        unsigned v = 0;
+#pragma unroll
+        for (int w = 0; w < 4; w++) v += (unsigned)lds_acc[w][reg][l];
+        const int val = (int)(v + offj * (unsigned)lds_rs[row] + colterm);
+        if (acc_out) acc_out[(long long)row * n + j] = val;
+        if (out) {
+            const float o = __builtin_fmaf((float)val, comb, col.bias);
+            out[(long long)row * n + j] = lds_rn[row] ? __builtin_nanf("") : o;
+        }
+    }
+}
+
+static osh_status run_minmax(const float *a, long long count, DqScratch *sc, int *nparts, hipStream_t st,
+                             int *zero = nullptr, int zero_n = 0) {
     long long blocks = (count / 4 + DQ_THREADS - 1) / DQ_THREADS;
     if (blocks < 1) blocks = 1;
     if (blocks > DQ_MINMAX_BLOCKS) blocks = DQ_MINMAX_BLOCKS;
-    OSH_LAUNCH(dqmm_minmax_kernel, dim3((unsigned)blocks), dim3(DQ_THREADS), 0, st, a, count, sc);
+    OSH_LAUNCH(dqmm_minmax_kernel, dim3((unsigned)blocks), dim3(DQ_THREADS), 0, st, a, count, sc, zero,
+               zero_n);
     *nparts = (int)blocks;
     OSH_LAUNCH_CHECK("dqmm_minmax_kernel");
+    return OSH_OK;
+}
+
+static osh_status launch_int8_gemm(int m, int k, int n, const int8_t *apk, const int8_t *wpk, const int *colsum,
+                                   const int *off, const int *rownan, const DqScratch *sc, const float *wscale,
+                                   int n_wscale, const float *bias, float *out, int *acc_out, hipStream_t st) {
+    const int mt = pad32(m) / 32, nb = (pad32(n) / 32 + 3) / 4;
+    if ((long long)mt * nb > 0x7fffffffLL) return fail(OSH_E_UNSUPPORTED, "int8 GEMM grid too large");
+#define OSH_I8_GEMM_OUT(TM, SETS, OUT)                                                                       \
+    OSH_LAUNCH((dqmm_gemm_kernel<TM, SETS, OUT>), dim3((unsigned)((long long)((mt + TM - 1) / TM) * nb)),    \
+               dim3(256), 0, st, m, k, n, apk, wpk, colsum, off, rownan, sc, wscale, n_wscale, bias, out, acc_out)
+#define OSH_I8_GEMM(TM, SETS)                                         \
+    do {                                                              \
+        if (!acc_out) OSH_I8_GEMM_OUT(TM, SETS, DQG_FLOAT);           \
+        else if (!out) OSH_I8_GEMM_OUT(TM, SETS, DQG_ACC);            \
+        else OSH_I8_GEMM_OUT(TM, SETS, DQG_FLOAT | DQG_ACC);          \
+    } while (0)
+    // 64-row tiles (half the W traffic) where they still give 3 workgroups for
+    // every 2 CUs, with two stages in flight so that more workgroups share a CU:
+    // 1028 x 1280 x 5120 26.2 us (32-row tiles 29.1); 669 x 352 x 2368 13.3 (12.8).
+    if ((long long)((mt + 1) / 2) * nb >= 3LL * device_cus() / 2) OSH_I8_GEMM(2, 2);
+    else OSH_I8_GEMM(1, 4);
+#undef OSH_I8_GEMM
+#undef OSH_I8_GEMM_OUT
+    OSH_LAUNCH_CHECK("dqmm_gemm_kernel");
     return OSH_OK;
 }
 
@@ -882,21 +1156,41 @@ static osh_status dqmm_run(int m, int k, int n, const float *d_a, const void *d_
                            int n_wscale, const float *d_bias, float *d_out, int32_t *d_acc, int32_t *d_qparams,
                            void *d_scratch, hipStream_t st) {
     DqScratch *sc = static_cast<DqScratch *>(d_scratch);
-    int *rowsum = reinterpret_cast<int *>(sc + 1);
-    int8_t *apk = reinterpret_cast<int8_t *>(rowsum + 2 * pad32(m));
+    int *rownan = reinterpret_cast<int *>(sc + 1);  // the second mpad ints of the layout are spare
+    int8_t *apk = reinterpret_cast<int8_t *>(rownan + 2 * pad32(m));
     const int8_t *frag = static_cast<const int8_t *>(d_wpacked);
     const int *colsum = reinterpret_cast<const int *>(frag + (size_t)pad32(n) * pad32(k));
     const int *off = colsum + pad32(n);
     const long long fblocks = (long long)((pad32(n) / 32 + DQF_WAVES - 1) / DQF_WAVES) * (pad32(m) / 32);
     const long long total = (long long)m * k;
     int nparts = 0;
-    osh_status r = run_minmax(d_a, total, sc, &nparts, st);
-    if (r != OSH_OK) return r;
     const bool full = m % 32 == 0 && n % 128 == 0 && k % (32 * DQF_KS) == 0 &&
                       (reinterpret_cast<uintptr_t>(d_a) & 15) == 0;
     const int variant = dqmm_variant();
-    if (variant != 1 && fblocks <= 0x7fffffffLL) {
-        if (full && variant == 0 && d_acc)
+    // Every 128-column block of the fused launch quantizes its rows again, which
+    // a separate quantize launch (about 4.3 us) ends: the two cross at about
+    // 1e9 products on ragged tiles (669 x 352 x 2368 11.4 us in two launches,
+    // 13.2 in three; 777 x 700 x 3000 22.3 and 17.7; 1028 x 1280 x 5120 44.4 and
+    // 26.2) and 4e9 on full ones (2048 x 512 x 2048 15.4 and 18.3; 1024 x 1024 x
+    // 4096 22.3 and 20.6).  At most 16 rows take the skinny kernel instead
+    // (16 x 2048 x 8192 14.3 us, 13.5 in three).
+    const double macs = (double)m * n * k;
+    const bool three = variant == 1 || fblocks > 0x7fffffffLL || (m > 16 && macs > (full ? 4e9 : 1e9));
+    osh_status r = run_minmax(d_a, total, sc, &nparts, st, three ? rownan : nullptr, three ? pad32(m) : 0);
+    if (r != OSH_OK) return r;
+    if (!three) {
+        if (m <= 16) {
+            const dim3 grid((unsigned)(pad32(n) / 32));
+#define OSH_SKINNY(RT)                                                                                               \
+    OSH_LAUNCH(dqmm_skinny_kernel<RT>, grid, dim3(256), 0, st, m, k, n, d_a, sc, nparts, (int *)d_qparams, frag, colsum, \
+               off, d_wscale, n_wscale, d_bias, d_out, (int *)d_acc)
+            if (m == 1) OSH_SKINNY(1);
+            else if (m == 2) OSH_SKINNY(2);
+            else if (m <= 4) OSH_SKINNY(4);
+            else if (m <= 8) OSH_SKINNY(8);
+            else OSH_SKINNY(16);
+#undef OSH_SKINNY
+        } else if (full && variant == 0 && d_acc)
             OSH_LAUNCH(dqmm_fused16_kernel<true>, dim3((unsigned)fblocks), dim3(64 * DQF_WAVES), 0, st, m, k, n,
                        d_a, sc, nparts, (int *)d_qparams, frag, colsum, off, d_wscale, n_wscale, d_bias, d_out,
                        (int *)d_acc);
@@ -916,14 +1210,15 @@ static osh_status dqmm_run(int m, int k, int n, const float *d_a, const void *d_
         t_dqmm_launches = 2;
         return OSH_OK;
     }
-    const int rows_per_block = DQ_THREADS / 64;
-    OSH_LAUNCH(dqmm_quantize_kernel, dim3((unsigned)((pad32(m) + rows_per_block - 1) / rows_per_block)),
-                       dim3(DQ_THREADS), 0, st, d_a, m, k, sc, nparts, (int *)d_qparams, rowsum, apk);
+    const long long waves = (long long)(pad32(m) / 32) * ((pad32(k) / 32 + DQ_QF - 1) / DQ_QF);
+    const long long qblocks = (waves + DQ_THREADS / 64 - 1) / (DQ_THREADS / 64);
+    if (qblocks > 0x7fffffffLL) return fail(OSH_E_UNSUPPORTED, "DQM: m too large");
+    OSH_LAUNCH(dqmm_quantize_kernel, dim3((unsigned)qblocks), dim3(DQ_THREADS), 0, st, d_a, m, k, sc, nparts,
+               (int *)d_qparams, rownan, apk);
     OSH_LAUNCH_CHECK("dqmm_quantize_kernel");
-    dim3 grid((pad32(n) / 32 + 1) / 2, (pad32(m) / 32 + 1) / 2);
-    OSH_LAUNCH(dqmm_gemm_kernel, grid, dim3(256), 0, st, m, k, n, apk, frag, colsum, off, rowsum, sc,
-                       d_wscale, n_wscale, d_bias, d_out, (int *)d_acc);
-    OSH_LAUNCH_CHECK("dqmm_gemm_kernel");
+    r = launch_int8_gemm(m, k, n, apk, frag, colsum, off, rownan, sc, d_wscale, n_wscale, d_bias, d_out, (int *)d_acc,
+                         st);
+    if (r != OSH_OK) return r;
     t_dqmm_launches = 3;
     return OSH_OK;
 }
@@ -1073,22 +1368,18 @@ OSH_API osh_status osh_matmul_integer(int m, int k, int n, const void *d_a, int 
     if (pad32(m) / 32 > 2 * 65535) return fail(OSH_E_UNSUPPORTED, "MatMulInteger: m too large");
     hipStream_t st = to_stream(s);
     DqScratch *sc = static_cast<DqScratch *>(d_scratch);
-    int *rowsum = reinterpret_cast<int *>(sc + 1);
-    int8_t *apk = reinterpret_cast<int8_t *>(rowsum + 2 * pad32(m));
-    const int rows_per_block = DQ_THREADS / 64;
-    OSH_LAUNCH(mmi_pack_a_kernel, dim3((unsigned)((pad32(m) + rows_per_block - 1) / rows_per_block)),
-                       dim3(DQ_THREADS), 0, st, static_cast<const uint8_t *>(d_a), m, k, a_signed, a_zp, sc, rowsum,
-                       apk);
+    int *rownan = reinterpret_cast<int *>(sc + 1);  // the second mpad ints of the layout are spare
+    int8_t *apk = reinterpret_cast<int8_t *>(rownan + 2 * pad32(m));
+    const long long waves = (long long)(pad32(m) / 32) * ((pad32(k) / 32 + DQ_MF - 1) / DQ_MF);
+    const long long pblocks = (waves + DQ_THREADS / 64 - 1) / (DQ_THREADS / 64);
+    if (pblocks > 0x7fffffffLL) return fail(OSH_E_UNSUPPORTED, "MatMulInteger: m too large");
+    OSH_LAUNCH(mmi_pack_a_kernel, dim3((unsigned)pblocks), dim3(DQ_THREADS), 0, st,
+               static_cast<const uint8_t *>(d_a), m, k, a_signed, a_zp, sc, rownan, apk);
     OSH_LAUNCH_CHECK("mmi_pack_a_kernel");
     const int8_t *frag = static_cast<const int8_t *>(d_wpacked);
     const int *colsum = reinterpret_cast<const int *>(frag + (size_t)pad32(n) * pad32(k));
     const int *off = colsum + pad32(n);
-    dim3 grid((pad32(n) / 32 + 1) / 2, (pad32(m) / 32 + 1) / 2);
-    OSH_LAUNCH(dqmm_gemm_kernel, grid, dim3(256), 0, st, m, k, n, apk, frag, colsum, off, rowsum, sc,
-                       static_cast<const float *>(nullptr), 1, static_cast<const float *>(nullptr),
-                       static_cast<float *>(nullptr), (int *)d_c);
-    OSH_LAUNCH_CHECK("dqmm_gemm_kernel");
-    return OSH_OK;
+    return launch_int8_gemm(m, k, n, apk, frag, colsum, off, rownan, sc, nullptr, 1, nullptr, nullptr, (int *)d_c, st);
 }
 
 OSH_API osh_status osh_dynamic_quantize_linear(int64_t n, const float *d_x, uint8_t *d_q, int32_t *d_qparams,

@@ -363,3 +363,52 @@ def _no_acc_case(cuda, oracle, m, k, n, noalloc, offset):
     good[m // 3] = False
     assert np.isnan(got[m // 3]).all()
     assert np.array_equal(got[good].view(np.uint32), eo[good].view(np.uint32))
+
+
+@pytest.mark.parametrize("m,k,n,wdt,variant,launches", [
+    # at most 16 rows: one workgroup per 32 columns, K split over its waves in passes of 1024
+    (1, 1, 1, np.int8, 0, 2), (2, 31, 33, np.uint8, 0, 2), (3, 1024, 32, np.int8, 0, 2), (4, 1025, 31, np.uint8, 0, 2),
+    (5, 2049, 65, np.int8, 0, 2), (8, 4097, 40, np.uint8, 0, 2), (9, 130, 513, np.int8, 0, 2),
+    (16, 2050, 96, np.uint8, 0, 2),
+    # ragged tiles of the fused launch: one past a tile, k % 4 != 0, two and three passes
+    (17, 36, 129, np.int8, 0, 2), (33, 513, 127, np.uint8, 0, 2), (65, 1100, 130, np.int8, 0, 2),
+    # three launches, 32-row tiles: one and several stages, ragged in each direction
+    (31, 33, 127, np.uint8, 1, 3), (33, 128, 129, np.int8, 1, 3), (65, 1157, 257, np.uint8, 1, 3),
+    # 64-row tiles (enough workgroups), and the size rule's own choice of three launches
+    (1000, 70, 3100, np.uint8, 1, 3), (1030, 801, 1300, np.int8, 0, 3),
+])
+def test_dqmm_tile_edges(cuda, oracle, m, k, n, wdt, variant, launches):
+    """Each route of the size rules at the edges of its tiles: accumulators and
+    outputs equal the oracle bit for bit, a NaN row stays NaN, and the range of
+    A is that of the other values."""
+    import ctypes as C
+    from onnxsharp_amd import native as N
+    print(f"dqmm edges m={m} k={k} n={n} w={wdt.__name__} variant={variant}", flush=True)
+    a = synth.normal(11 * m + k, (m, k))
+    if m > 1:
+        a[m // 2, k - 1] = np.nan
+    lo, hi, base = (-128, 127, 0) if wdt == np.int8 else (0, 255, 128)
+    w = synth.randint(m + 5 * n, (k, n), lo, hi, wdt)
+    wzp = synth.randint(n, (n,), -20, 20, np.int32) + base
+    ws = synth.uniform(k + 5 * n, (n,), 0.001, 0.02)
+    bias = synth.normal(m + n + 1, (n,), 0, 0.01)
+    old, nl = C.c_int(), C.c_int()
+    N.call("osh_config_get", b"dqmm_variant", C.byref(old))
+    try:
+        N.call("osh_config_set", b"dqmm_variant", variant)
+        out, acc, s, z = run_dqmm(cuda, a, w, wzp, ws, bias)
+        N.call("osh_config_get", b"dqmm_launches", C.byref(nl))
+    finally:
+        N.call("osh_config_set", b"dqmm_variant", old.value)
+    assert nl.value == launches
+    clean = a.copy()
+    if m > 1:
+        clean[m // 2, k - 1] = 0.0
+        assert np.isnan(out[m // 2]).all()
+    eo, eacc, _, es, ez = oracle.dqmm(clean, w, wzp, ws, bias)
+    assert (s, z) == (es, ez)
+    good = np.ones(m, bool)
+    if m > 1:
+        good[m // 2] = False
+    assert np.array_equal(acc[good], eacc[good])
+    assert np.array_equal(out[good], eo[good])
