@@ -191,15 +191,151 @@ __global__ __launch_bounds__(256) void dw3_conv_kernel(osh_conv_params p, const 
     dw3_conv_at<ACT, S>(p, x, w, bias, res, y, blockIdx.x * 256 + threadIdx.x);
 }
 
+
+// K x K depthwise, dilation 1, stride S, left pad K / 2: four neighbouring
+// outputs of R rows a thread.  One output a thread spends most of its time on
+// index arithmetic and nine separate loads (4 x 128 x 112 x 112: 25.9 us, 2.0
+// TB/s); here a thread loads the 3 S + K columns under its strip once for all
+// four outputs (and, between its rows, once for both): the left halo one by
+// one, the rest, which starts at the strip's own column, 16 bytes at a time;
+// and it stores 16 bytes (12.5 us, 4.1 TB/s of the 4.75 a large copy reaches).
+// What lies outside the tensor loads as zero through
+// the buffer descriptor; taps off the map are skipped in the chain, as in
+// dw_conv_at.
+template <int ACT, int K, int S, int R>
+__device__ __forceinline__ void dws_conv_at(const osh_conv_params &p, const float *__restrict__ x,
+                                            const float *__restrict__ w, const float *__restrict__ bias,
+                                            const float *__restrict__ res, float *__restrict__ y, unsigned idx) {
+    constexpr int H = K / 2;          // left halo
+    constexpr int NC = 3 * S + K;     // input columns under the strip
+    constexpr int NQ = (NC - H) / 4;  // 16-byte loads a row, then single columns
+    constexpr int NR = (R - 1) * S + K;  // input rows
+    const unsigned sx = (unsigned)(p.ow + 3) / 4, sy = (unsigned)(p.oh + R - 1) / R;
+    const unsigned planes = (unsigned)p.n * p.m;
+    const unsigned t = idx / sx;
+    const int ox0 = (int)(idx - t * sx) * 4;
+    const unsigned plane = t / sy;
+    const int oy0 = (int)(t - plane * sy) * R;
+    if (plane >= planes) return;
+    const unsigned c = plane % (unsigned)p.m;
+    __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, (int)(planes * (unsigned)(p.h * p.w) * 4u), 0x00020000);
+    const int iy0 = oy0 * S - p.pt, ix0 = ox0 * S - H;
+    float v[NR][NC];
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const int iy = iy0 + r;
+        // a row off the map loads past the tensor's end (which is below 2^31 - 64)
+        const int at = (unsigned)iy < (unsigned)p.h
+                           ? (int)(((plane * (unsigned)p.h + (unsigned)iy) * (unsigned)p.w + (unsigned)(ox0 * S)) * 4u)
+                           : 0x7fffffc0;
+#pragma unroll
+        for (int i = 0; i < H; i++) v[r][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, at - 4 * (H - i), 0, 0));
+#pragma unroll
+        for (int l = 0; l < NQ; l++) {
+            const auto q = __builtin_amdgcn_raw_buffer_load_b128(rx, at + 16 * l, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[r][H + 4 * l + e] = __uint_as_float(q[e]);
+        }
+#pragma unroll
+        for (int i = H + 4 * NQ; i < NC; i++) v[r][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, at + 4 * (i - H), 0, 0));
+    }
+    float wv[K * K];
+#pragma unroll
+    for (int i = 0; i < K * K; i++) wv[i] = w[c * (K * K) + i];
+    const float b = bias ? bias[c] : 0.f;
+    const unsigned o0 = (plane * (unsigned)p.oh + (unsigned)oy0) * (unsigned)p.ow + (unsigned)ox0;
+    __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)y, (short)0, (int)(planes * (unsigned)(p.oh * p.ow) * 4u), 0x00020000);
+    float rv[R][4];
+    if (res) {  // read past the strip's end stays inside the residual or gives zeros
+        __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)res, (short)0, (int)(planes * (unsigned)(p.oh * p.ow) * 4u), 0x00020000);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const auto q = __builtin_amdgcn_raw_buffer_load_b128(rr, (int)((o0 + r * (unsigned)p.ow) * 4u), 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) rv[r][e] = __uint_as_float(q[e]);
+        }
+    }
+    bool cin[NC];
+#pragma unroll
+    for (int i = 0; i < NC; i++) cin[i] = (unsigned)(ix0 + i) < (unsigned)p.w;
+    float acc[R][4];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[r][e] = b;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int ky = 0; ky < K; ky++)
+            if ((unsigned)(iy0 + r * S + ky) < (unsigned)p.h) {
+#pragma unroll
+                for (int kx = 0; kx < K; kx++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float f = __builtin_fmaf(wv[ky * K + kx], v[r * S + ky][e * S + kx], acc[r][e]);
+                        acc[r][e] = cin[e * S + kx] ? f : acc[r][e];
+                    }
+            }
+    const int live = p.ow - ox0;  // outputs of the strip inside the row
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (oy0 + r >= p.oh) break;
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            o[e] = activate<ACT>(acc[r][e]);
+            if (res) o[e] += rv[r][e];
+        }
+        const int at = (int)((o0 + r * (unsigned)p.ow) * 4u);
+        if (live >= 4) {
+            typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(o[0]), __float_as_uint(o[1]),
+                                                         __float_as_uint(o[2]), __float_as_uint(o[3])},
+                                                   ry, at, 0, 0);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; e++)
+                if (e < live) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[e]), ry, at + 4 * e, 0, 0);
+        }
+    }
+}
+
+template <int ACT, int K, int S, int R>
+__global__ __launch_bounds__(256) void dws_conv_kernel(osh_conv_params p, const float *__restrict__ x,
+                                                       const float *__restrict__ w, const float *__restrict__ bias,
+                                                       const float *__restrict__ res, float *__restrict__ y) {
+    dws_conv_at<ACT, K, S, R>(p, x, w, bias, res, y, blockIdx.x * 256 + threadIdx.x);
+}
+
+// Below this many outputs a 3 x 3 conv keeps one output a thread, which has
+// four times the waves to hide its one round trip with: 256 x 20 x 20 2.75 us
+// (strips 2.91), 32 x 64 x 64 2.77 (2.94), 128 x 40 x 40 3.19 (2.95).  5 x 5 has only the general loop to
+// lose (224 x 14 x 76 6.6 us, strips 3.7).
+constexpr long long DWS_MIN_OUTPUTS = 160000;
+
+// Kernels of 3 and 5, one stride of 1 or 2 in both directions, no dilation,
+// tensors whose byte offsets fit 31 bits.
+inline bool dws_eligible(const osh_conv_params *p) {
+    return (p->kh == 3 || p->kh == 5) && p->kw == p->kh && p->dh == 1 && p->dw == 1 && p->pl == p->kw / 2 &&
+           p->sh == p->sw && (p->sh == 1 || p->sh == 2) && (long long)p->n * p->m * p->oh * p->ow * 4 < (1LL << 31) - 64 &&
+           (long long)p->n * p->c * p->h * p->w * 4 < (1LL << 31) - 64;
+}
+
 // Several depthwise convs in one launch: workgroup b covers outputs
-// 256 (b - start[i]) .. of conv i (ConvGroup's block table).  S > 0: every
-// member is a 3x3 stride-S conv (dw3_eligible).
+// 256 (b - start[i]) .. of conv i (ConvGroup's block table), with S = 3 strips
+// of four outputs.  S = 1, 2: every member is a 3x3 stride-S conv (dw3_eligible).
 template <int ACT, int S>
 __global__ __launch_bounds__(256) void dw_conv_group_kernel(ConvGroup g) {
     const int b = blockIdx.x;
     int i = 0;
     while (i + 1 < g.count && b >= g.start[i + 1]) i++;
-    if constexpr (S > 0)
+    if constexpr (S == 3)  // 3x3 stride 1 in strips (dws_eligible)
+        dws_conv_at<ACT, 3, 1, 1>(g.p[i], g.x[i], g.w[i], g.bias[i], g.res[i], g.y[i],
+                                  (b - g.start[i]) * 256 + threadIdx.x);
+    else if constexpr (S > 0)
         dw3_conv_at<ACT, S>(g.p[i], g.x[i], g.w[i], g.bias[i], g.res[i], g.y[i], (b - g.start[i]) * 256 + threadIdx.x);
     else
         dw_conv_at<ACT>(g.p[i], g.x[i], g.w[i], g.bias[i], g.res[i], g.y[i],
@@ -827,6 +963,31 @@ static osh_status conv2d(const osh_conv_params *p, const float *d_x, const void 
     case ALGO_DEPTHWISE: {
         long long total = (long long)p->n * p->m * out_hw;
         dim3 grid((unsigned)((total + 255) / 256));
+        if (dws_eligible(p) && (p->kh == 5 || total >= DWS_MIN_OUTPUTS)) {
+            // Rows a thread: more of them share loads, fewer of them keep more
+            // waves in flight.  Stride 1: 4 x 128 x 112 x 112 18.9, 15.2, 14.3
+            // us with 1, 2, 4 rows, 32 x 160 x 160 4.63, 4.28, 4.54, 64 x 80 x 80
+            // 3.46, 3.53, 4.42; stride 2 (rows share less): 4 x 128 x 112 x 112
+            // 7.1, 7.2, 7.5.
+            const int rows = p->sh == 2 || total < 800000 ? 1 : (p->kh == 5 || total < 4000000 ? 2 : 4);
+            const long long threads = (long long)p->n * p->m * ((p->oh + rows - 1) / rows) * ((p->ow + 3) / 4);
+            grid.x = (unsigned)((threads + 255) / 256);
+#define OSH_DWS(K, S, R)                                                                                               \
+    do {                                                                                                               \
+        OSH_DISPATCH_ACT(act, ACT, OSH_LAUNCH((dws_conv_kernel<ACT, K, S, R>), grid, dim3(256), 0, stream, *p, d_x, w, \
+                                              d_bias, d_res, d_y));                                                    \
+    } while (0)
+            if (p->kh == 3 && p->sh == 2) OSH_DWS(3, 2, 1);
+            else if (p->kh == 3 && rows == 1) OSH_DWS(3, 1, 1);
+            else if (p->kh == 3 && rows == 2) OSH_DWS(3, 1, 2);
+            else if (p->kh == 3) OSH_DWS(3, 1, 4);
+            else if (p->sh == 2) OSH_DWS(5, 2, 1);
+            else if (rows == 1) OSH_DWS(5, 1, 1);
+            else OSH_DWS(5, 1, 2);
+#undef OSH_DWS
+            OSH_LAUNCH_CHECK("dws_conv_kernel");
+            return OSH_OK;
+        }
         if (dw3_eligible(p)) {
             if (p->sh == 1) {
                 OSH_DISPATCH_ACT(act, ACT,
@@ -976,17 +1137,28 @@ static osh_status conv2d_group(int count, const osh_conv_params *ps, const float
         g.y[k] = ys[i];
     }
     if (a0 == ALGO_DEPTHWISE) {
-        long long total = 0;
+        int s3 = dw3_eligible(&ps[0]) ? ps[0].sh : 0;  // every member 3x3 at one stride: the 3x3 path
+        long long outputs = 0;
+        bool strips = s3 == 1;  // and enough outputs for strips of four a thread
         for (int i = 0; i < count; i++) {
-            g.start[i] = (int)total;
-            total += ((long long)ps[i].n * ps[i].m * ps[i].oh * ps[i].ow + 255) / 256;
+            if (!dw3_eligible(&ps[i]) || ps[i].sh != s3) s3 = 0;
+            strips = strips && s3 == 1 && ps[i].kh == 3 && dws_eligible(&ps[i]);
+            outputs += (long long)ps[i].n * ps[i].m * ps[i].oh * ps[i].ow;
+        }
+        strips = strips && outputs >= DWS_MIN_OUTPUTS;
+        long long total = 0;
+        for (int k = 0; k < count; k++) {
+            const osh_conv_params &p = g.p[k];
+            g.start[k] = (int)total;
+            total += ((long long)p.n * p.m * p.oh * (strips ? (p.ow + 3) / 4 : p.ow) + 255) / 256;
             if (total > 0x7fffffffLL) return fail(OSH_E_UNSUPPORTED, "Conv group: grid too large");
         }
         g.start[count] = (int)total;
-        int s3 = dw3_eligible(&ps[0]) ? ps[0].sh : 0;  // every member 3x3 at one stride: the 3x3 path
-        for (int i = 1; i < count; i++)
-            if (!dw3_eligible(&ps[i]) || ps[i].sh != s3) s3 = 0;
-        if (s3 == 1) {
+        if (strips) {
+            OSH_DISPATCH_ACT(act, ACT,
+                             OSH_LAUNCH((dw_conv_group_kernel<ACT, 3>), dim3((unsigned)total), dim3(256), 0, st,
+                                                g));
+        } else if (s3 == 1) {
             OSH_DISPATCH_ACT(act, ACT,
                              OSH_LAUNCH((dw_conv_group_kernel<ACT, 1>), dim3((unsigned)total), dim3(256), 0, st,
                                                 g));

@@ -893,3 +893,72 @@ def test_conv_without_nchwc_follows_the_avx2_dispatch(cuda, oracle, name, xs, ws
     assert np.array_equal(y, ref), f"max |d| {np.abs(y - ref).max():.3e} at {np.argwhere(y != ref)[:3]}"
     # and not the NCHWc chain's bits (the two orders round differently here)
     assert not np.array_equal(y, oracle_conv(oracle, x, w, b, p, "Silu", nchwc=1))
+
+
+DW_STRIP_CASES = [
+    # (x shape, K, stride, pads, residual): strips of four outputs, 1/2/4 rows a thread
+    ((1, 4, 1, 1), 5, 1, 2, False), ((2, 3, 5, 6), 5, 2, 2, True), ((1, 7, 9, 3), 5, 1, 2, False),
+    ((1, 20, 91, 91), 3, 1, 1, True),     # 165620 outputs: one row
+    ((3, 24, 61, 62), 3, 2, 1, False),    # stride 2, below the strips' minimum
+    ((3, 60, 61, 62), 3, 2, 1, True),     # stride 2 strips: 172980 outputs
+    ((2, 31, 115, 117), 3, 1, 1, False),  # two rows, odd height and width
+    ((1, 40, 143, 142), 5, 1, 2, True),   # 5x5, two rows
+    ((5, 64, 113, 115), 3, 1, 1, True),   # four rows, odd height and width
+    ((1, 20, 90, 90), 3, 1, 0, False),    # a left pad other than K / 2: one output a thread
+]
+
+
+@pytest.mark.parametrize("xs,k,s,pad,residual", DW_STRIP_CASES, ids=[f"{c[0]}_k{c[1]}s{c[2]}p{c[3]}" for c in DW_STRIP_CASES])
+def test_depthwise_strips_are_the_depthwise_chain(cuda, oracle, xs, k, s, pad, residual):
+    """Depthwise convs at the edges of their strips (widths and heights that
+    are no multiples of a strip, planes side by side) are the ky -> kx chain
+    bit for bit; an infinite weight meets taps off the map nowhere (inf * 0
+    would be a NaN), and a NaN in the input reaches only its own windows."""
+    import torch
+    from onnxsharp_amd.layers import ConvLayer
+    print(f"depthwise strips x={xs} k={k} s={s} p={pad}", flush=True)
+    c = xs[1]
+    seed = sum(xs) * 13 + k
+    x = synth.uniform(seed, xs, -1, 1)
+    x.reshape(-1)[x.size // 2] = np.nan
+    w = synth.normal(seed + 1, (c, 1, k, k), 0, 0.2)
+    w[0, 0, 0, 0] = np.inf
+    x[:, 0] = np.abs(x[:, 0]) + 0.5
+    b = synth.normal(seed + 2, (c,), 0, 0.01)
+    layer = ConvLayer(group=c, strides=[s, s], pads=[pad] * 4, fused_activation="Relu")
+    p = layer.resolve(xs, w.shape)
+    r = synth.normal(seed + 3, (p.n, p.m, p.oh, p.ow), 0, 1) if residual else None
+    y = layer.forward(_t(x, cuda), _t(w, cuda), _t(b, cuda), residual=None if r is None else _t(r, cuda)).cpu().numpy()
+    ref = oracle.relu(oracle.conv_reference(x, w, b, (s, s), (pad, pad), (1, 1), c, (p.oh, p.ow)))
+    if r is not None:
+        ref = ref + r
+    assert np.array_equal(y, ref, equal_nan=True), f"max |d| {np.nanmax(np.abs(y - ref)):.3e}"
+
+
+def test_depthwise_group_in_strips(cuda):
+    """A depthwise group with enough outputs for strips, and one whose members
+    have different kernels, equal the convs launched one by one."""
+    import torch
+    from onnxsharp_amd import native as N
+    from onnxsharp_amd.layers import ConvLayer
+    for shapes in ([((1, 18, 90, 91), 3), ((1, 24, 33, 34), 3), ((2, 8, 7, 5), 3)], [((1, 16, 20, 21), 3), ((1, 8, 30, 30), 5)]):
+        print(f"depthwise group {shapes}", flush=True)
+        ps, xs, ws, bs, ys, want, keep = [], [], [], [], [], [], []
+        for i, (sh, k) in enumerate(shapes):
+            c = sh[1]
+            x = _t(synth.uniform(70 + i, sh, -1, 1), cuda)
+            w = _t(synth.normal(80 + i, (c, 1, k, k), 0, 0.2), cuda)
+            b = _t(synth.normal(90 + i, (c,), 0, 0.01), cuda)
+            layer = ConvLayer(group=c, pads=[k // 2] * 4, fused_activation="Silu")
+            want.append(layer.forward(x, w, b))
+            p, packed = layer.prepack_weights(sh, w)
+            y = torch.full_like(want[-1], float("nan"))
+            ps.append(p), xs.append(x), ws.append(packed), bs.append(b), ys.append(y), keep.append(layer)
+        n = len(ps)
+        arr = lambda ts: (C.c_void_p * n)(*[t.data_ptr() for t in ts])
+        st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        N.call("osh_conv2d_group_f32", n, (N.ConvParams * n)(*ps), arr(xs), arr(ws), arr(bs), N.ACT_SILU, None, arr(ys),
+               st)
+        torch.cuda.synchronize()
+        for y, e in zip(ys, want):
+            assert torch.equal(y, e)
