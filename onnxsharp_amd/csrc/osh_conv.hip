@@ -1059,14 +1059,33 @@ static osh_status conv2d(const osh_conv_params *p, const float *d_x, const void 
             },
             stream);
     case ALGO_WINOGRAD: {
-        const long long tiles = (long long)p->n * ((p->h + 1) / 2) * ((p->w + 1) / 2);
-        dim3 grid((unsigned)((p->m + 15) / 16), (unsigned)((tiles + 15) / 16));
-        if (grid.y > 65535) return fail(OSH_E_UNSUPPORTED, "Conv: Winograd grid too large");
         const float4 *u = reinterpret_cast<const float4 *>(d_wpacked);
-        OSH_DISPATCH_ACT(act, ACT,
-                         OSH_LAUNCH(wino_f23_kernel<ACT>, grid, dim3(256), 0, stream, *p, d_x, u, d_bias,
-                                            d_res, d_y));
-        OSH_LAUNCH_CHECK("wino_f23_kernel");
+#define OSH_WINO(OB)                                                                                              \
+    do {                                                                                                          \
+        dim3 grid((unsigned)((p->m + 16 * OB - 1) / (16 * OB)), (unsigned)((tiles + 15) / 16));                   \
+        OSH_DISPATCH_ACT(act, ACT, OSH_LAUNCH((wino_f23_kernel<ACT, OB>), grid, dim3(256 * OB), 0, stream, q, xi, \
+                                              u, d_bias, ri, yi));                                                \
+    } while (0)
+        // all images in one launch while those of one workgroup (at most
+        // three: a map has nine tiles or more) stay within 31 bits, else one by one
+        const long long xi_bytes = (long long)p->c * p->h * p->w * 4;
+        const int step = p->n == 1 || 4 * xi_bytes < kWinoNowhere ? p->n : 1;
+        for (int i = 0; i < p->n; i += step) {
+            osh_conv_params q = *p;
+            q.n = step;
+            const float *xi = d_x + i * (xi_bytes / 4);
+            const float *ri = d_res ? d_res + (long long)i * p->m * out_hw : nullptr;
+            float *yi = d_y + (long long)i * p->m * out_hw;
+            const long long tiles = (long long)step * ((p->h + 1) / 2) * ((p->w + 1) / 2);
+            // Two output blocks a workgroup where that still gives most CUs
+            // one: 8 x 256 x 14 x 14 -> 256 (200 workgroups) 18.6 us (one block
+            // 21.1), 2 x 64 x 13 x 74 -> 200 (231) 7.9 (9.0); 2 x 128 x 28 x 28 ->
+            // 128 (100) 10.9 (9.0).
+            if (p->m > 16 && (tiles + 15) / 16 * ((p->m + 31) / 32) >= 5 * device_cus() / 8) OSH_WINO(2);
+            else OSH_WINO(1);
+            OSH_LAUNCH_CHECK("wino_f23_kernel");
+        }
+#undef OSH_WINO
         return OSH_OK;
     }
     case ALGO_PW16: {

@@ -16,16 +16,25 @@
 // columns past the last full 8-column vector of a partial 16-column panel
 // with separate multiply and add).
 //
-// One workgroup (4 waves) owns 16 output channels x 16 tiles (a tile is a
-// 2x2 output block; tiles run over batch, tile row, tile column) for all 16
-// components.  Per chunk of 16 input channels its 256 threads each transform
-// one (ic, tile) patch into LDS as [comp][ic 16][tile 16]; wave w runs the
-// MFMA chains of components 4w .. 4w+3 (the B operand of a k4 step is 64
-// consecutive floats of one component).  The input patches are loaded two
-// chunks ahead, the weight fragments likewise, and the component planes are
-// double-buffered.  At the end the accumulators go through LDS as
-// [comp][oc 16][tile 16] and each thread transforms one (oc, tile) to its 2x2
-// outputs.
+// One workgroup owns 16 tiles (a tile is a 2x2 output block; tiles run over
+// batch, tile row, tile column) x 16 OB output channels for all 16 components,
+// four waves an output block.  Per chunk of 16 input channels the first four
+// waves transform one (ic, tile) patch a thread into LDS as [comp][ic][tile];
+// wave w runs the MFMA chains of components 4 (w % 4) .. + 3 of output block
+// w / 4.  Patches and weights are loaded a chunk ahead of their use, all
+// without a condition (what does not exist lies outside the buffer descriptors
+// and loads as zero), a patch row as one value and three; the component planes
+// are double-buffered.  At the end the accumulators go through LDS as
+// [comp][oc][tile] and each thread transforms one (oc, tile) to its 2x2
+// outputs, stored two at a time.
+//
+// Bound by what the L2s deliver: 8 x 64 x 56 x 56 -> 64 with a residual reads
+// 215 MB through L1 with one output block a workgroup (weights once per 16
+// tiles, patches once per 16 channels), 160 with two, at about 15 TB/s: 24.1
+// and 22.9 us (31.9 before, its patch loads and stores one guarded value at a
+// time).  Workgroups of 32 tiles (weights shared through L1) 26.5 and 24.0; all
+// 16 components x 32 x 32 in four waves 33.6 (registers); patches two chunks
+// ahead no change.
 #pragma once
 
 #include "osh_common.h"
@@ -81,134 +90,188 @@ __global__ void wino_pack_kernel(int M, int C, const float *__restrict__ w, floa
         out[((((long long)comp * ocbs + ob) * cbs + cb) * 64 + lane) * 4 + slot] = u[comp];
 }
 
-struct WinoPatch {
-    float d[16];
-};
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
-template <int ACT>
-__global__ __launch_bounds__(256) void wino_f23_kernel(osh_conv_params p, const float *__restrict__ x,
-                                                       const float4 *__restrict__ up,
-                                                       const float *__restrict__ bias,
-                                                       const float *__restrict__ res, float *__restrict__ y) {
-    __shared__ __attribute__((aligned(16))) float vs[2][16 * 256];  // [buf][comp][ic 16][tile 16]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int C = p.c, H = p.h, W = p.w, M = p.m;
+// Buffer records end at least 64 bytes below this offset: a load there is zero.
+constexpr int kWinoNowhere = 0x7fffff80;
+
+template <int ACT, int OB>
+__global__ __launch_bounds__(256 * OB, 4) void wino_f23_kernel(osh_conv_params p, const float *__restrict__ x,
+                                                                   const float4 *__restrict__ up,
+                                                                   const float *__restrict__ bias,
+                                                                   const float *__restrict__ res,
+                                                                   float *__restrict__ y) {
+    static_assert(OB <= 2, "the accumulators take the two buffers of planes");
+    constexpr int NT = 16;                // tiles
+    constexpr int PLANE = 16 * NT;        // floats of one component's [ic 16][tile]
+    constexpr int MPLANE = 16 * OB * NT;  // floats of one component's [oc][tile]
+    __shared__ __attribute__((aligned(16))) float lds[2][16 * PLANE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int C = p.c, H = p.h, W = p.w, M = p.m, HW = H * W;
     const int tilesX = (W + 1) >> 1, tilesY = (H + 1) >> 1, T = tilesX * tilesY;
     const int ocbs = (M + 15) >> 4, cbs = (C + 15) >> 4;
-    const int ob = blockIdx.x;
-    // thread role for the transforms: (channel row tid >> 4, tile tid & 15)
-    const int row = tid >> 4, tl = tid & 15;
-    const long long tg = (long long)blockIdx.y * 16 + tl;
-    const bool tile_ok = tg < (long long)p.n * T;
-    int img = 0, ty = 0, tx = 0;
-    if (tile_ok) {
-        img = (int)(tg / T);
-        const int t = (int)(tg % T);
-        ty = t / tilesX;
-        tx = t - ty * tilesX;
+    const int ob = blockIdx.x * OB + (wave >> 2);
+    const bool transforms = wave < 4;  // the waves that transform patches (uniform)
+    // thread role: tile tid % NT, channel (of a chunk, then of the outputs) tid / NT
+    const int row = tid / NT, tl = tid % NT;
+    const unsigned tg = blockIdx.y * (unsigned)NT + tl;  // n * T fits 31 bits (winograd_eligible)
+    const unsigned imgb = blockIdx.y * (unsigned)NT / (unsigned)T;  // the workgroup's first image
+    const unsigned img = tg / (unsigned)T, tr = tg - img * (unsigned)T;
+    const int ty = (int)(tr / (unsigned)tilesX), tx = (int)tr - ty * tilesX;
+    const bool tile_ok = img < (unsigned)p.n;
+    // byte offsets of the patch rows at column 2 tx, from channel 0 of the
+    // chunk in the workgroup's first image (the host keeps the images of one
+    // workgroup within 31 bits)
+    int off[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int yy = 2 * ty - 1 + i;
+        off[i] = tile_ok && (unsigned)yy < (unsigned)H
+                     ? ((((int)(img - imgb) * C + row) * H + yy) * W + 2 * tx) * 4
+                     : kWinoNowhere;
     }
-    const int y0 = 2 * ty - 1, x0 = 2 * tx - 1;
-    const float *xin = x + (long long)img * C * H * W;
+    const bool in0 = tx > 0, in2 = 2 * tx + 1 < W, in3 = 2 * tx + 2 < W;
+    const long long xtotal = (long long)p.n * C * HW;
 
-    auto load_patch = [&](int cb) {
-        WinoPatch q;
-        const int ic = cb * 16 + row;
-        const bool ok = tile_ok && ic < C;
-        const float *xc = xin + (long long)(ok ? ic : 0) * H * W;
+    struct Patch {
+        float d[16];
+    };
+    auto load_patch = [&](Patch &q, int ch) {
+        const int c0 = ch * 16;
+        const long long at = ((long long)imgb * C + c0) * HW;
+        const long long rest = c0 < C ? (xtotal - at) * 4 : 0;
+        __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(x + (c0 < C ? at : 0)), (short)0, rest > kWinoNowhere - 64 ? kWinoNowhere - 64 : (int)rest,
+            0x00020000);
+        const bool ok = c0 + row < C;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int yy = y0 + i;
-            const bool rok = ok && yy >= 0 && yy < H;
+            const int o = ok ? off[i] : kWinoNowhere;
+            q.d[4 * i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, o - 4, 0, 0));
+            const auto v = __builtin_amdgcn_raw_buffer_load_b96(rx, o, 0, 0);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int xx = x0 + j;
-                q.d[i * 4 + j] = (rok && xx >= 0 && xx < W) ? xc[(long long)yy * W + xx] : 0.0f;
-            }
+            for (int e = 0; e < 3; e++) q.d[4 * i + 1 + e] = __uint_as_float(v[e]);
         }
-        return q;
     };
-    // V = B^T d B, stored at [comp][row][tl]
-    auto transform_store = [&](const WinoPatch &q, float *vb) {
-        float t[16];
+    // V = B^T d B (columns off the map zero), stored at [comp][row][tl]
+    auto transform_store = [&](const Patch &q, float *vb) {
+        float d[16], t[16];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            d[4 * i] = in0 ? q.d[4 * i] : 0.0f;
+            d[4 * i + 1] = q.d[4 * i + 1];
+            d[4 * i + 2] = in2 ? q.d[4 * i + 2] : 0.0f;
+            d[4 * i + 3] = in3 ? q.d[4 * i + 3] : 0.0f;
+        }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const float d0 = q.d[j], d1 = q.d[4 + j], d2 = q.d[8 + j], d3 = q.d[12 + j];
+            const float d0 = d[j], d1 = d[4 + j], d2 = d[8 + j], d3 = d[12 + j];
             t[j] = d0 - d2;
             t[4 + j] = d1 + d2;
             t[8 + j] = d2 - d1;
             t[12 + j] = d1 - d3;
         }
-        float *dst = vb + row * 16 + tl;
+        float *dst = vb + tid;  // row * NT + tl
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const float a = t[i * 4], b = t[i * 4 + 1], c2 = t[i * 4 + 2], d3 = t[i * 4 + 3];
-            dst[(i * 4) * 256] = a - c2;
-            dst[(i * 4 + 1) * 256] = b + c2;
-            dst[(i * 4 + 2) * 256] = c2 - b;
-            dst[(i * 4 + 3) * 256] = b - d3;
+            const float e0 = t[i * 4], e1 = t[i * 4 + 1], e2 = t[i * 4 + 2], e3 = t[i * 4 + 3];
+            dst[(i * 4) * PLANE] = e0 - e2;
+            dst[(i * 4 + 1) * PLANE] = e1 + e2;
+            dst[(i * 4 + 2) * PLANE] = e2 - e1;
+            dst[(i * 4 + 3) * PLANE] = e1 - e3;
         }
     };
-    // weight fragments of this wave's four components for chunk cb
-    const float4 *ub = up + (long long)ob * cbs * 64 + lane;
-    const long long ucomp = (long long)ocbs * cbs * 64;
-    auto load_u = [&](int cb, float4 u[4]) {
+    // weight fragments of this wave's four components and output block; an
+    // output block past the last has no descriptor and chunks past it lie
+    // outside: zeros
+    struct Weights {
+        f32x4 u[4];
+    };
+    __amdgpu_buffer_rsrc_t ru[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) u[q] = ub[(4 * wave + q) * ucomp + (long long)cb * 64];
+    for (int q = 0; q < 4; q++)
+        ru[q] = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(up + ((long long)(4 * (wave & 3) + q) * ocbs + (ob < ocbs ? ob : 0)) * cbs * 64), (short)0,
+            ob < ocbs ? cbs * 1024 : 0, 0x00020000);
+    auto load_u = [&](Weights &w, int ch) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(ru[q], lane * 16 + ch * 1024, 0, 0);
+            w.u[q] = f32x4{__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3])};
+        }
     };
 
     f32x4 acc[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    WinoPatch p0 = load_patch(0), p1;
-    float4 u0[4], u1[4], u2[4];
-    load_u(0, u0);
-    if (cbs > 1) {
-        p1 = load_patch(1);
-        load_u(1, u1);
+    auto multiply = [&](const Weights &w, const float *vs) {
+        const float *vb = vs + 4 * (wave & 3) * PLANE + lane;  // B operand: V[k = 4 s + lane >> 4][tile lane & 15]
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.u[q][s], vb[q * PLANE + 4 * s * NT], acc[q], 0, 0, 0);
+    };
+    Patch pa;
+    Weights w0, w1;
+    if (transforms) load_patch(pa, 0);
+    load_u(w0, 0);
+    if (transforms) {
+        transform_store(pa, lds[0]);
+        load_patch(pa, 1);
     }
-    transform_store(p0, vs[0]);
+    load_u(w1, 1);
     __syncthreads();
-    const int boff = (lane >> 4) * 16 + (lane & 15);  // B operand: V[k = lane >> 4][tile = lane & 15]
-    for (int cb = 0; cb < cbs; cb++) {
-        const int buf = cb & 1;
-        const bool pre = cb + 2 < cbs;
-        if (pre) {
-            p0 = load_patch(cb + 2);
-            load_u(cb + 2, u2);
+    for (int ch = 0; ch < cbs; ch += 2) {
+        // planes of chunk ch in buffer 0; pa and w1 hold chunk ch + 1
+        multiply(w0, lds[0]);
+        load_u(w0, ch + 2);
+        if (transforms) {
+            transform_store(pa, lds[1]);
+            load_patch(pa, ch + 2);
         }
-        const float *vb = vs[buf] + 4 * wave * 256 + boff;
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float a = s == 0 ? u0[q].x : s == 1 ? u0[q].y : s == 2 ? u0[q].z : u0[q].w;
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vb[q * 256 + s * 64], acc[q], 0, 0, 0);
-            }
-        }
-        if (cb + 1 < cbs) transform_store(p1, vs[buf ^ 1]);
         __syncthreads();
-        p1 = p0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            u0[q] = u1[q];
-            u1[q] = u2[q];
+        if (ch + 1 >= cbs) break;
+        multiply(w1, lds[1]);
+        load_u(w1, ch + 3);
+        if (transforms) {
+            transform_store(pa, lds[0]);
+            load_patch(pa, ch + 3);
         }
+        __syncthreads();
     }
-    // accumulators -> [comp][oc 16][tile 16]; D[row 4g + r][col j]
+    // accumulators -> [comp][oc][tile]; D[row 4g + r][col j]
+    float *ms = lds[0];
     {
-        float *ms = vs[0] + 4 * wave * 256 + (lane >> 4) * 64 + (lane & 15);
+        float *d = ms + 4 * (wave & 3) * MPLANE + (16 * (wave >> 2) + 4 * (lane >> 4)) * NT + (lane & 15);
 #pragma unroll
         for (int q = 0; q < 4; q++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) ms[q * 256 + r * 16] = acc[q][r];
+            for (int r = 0; r < 4; r++) d[q * MPLANE + r * NT] = acc[q][r];
+    }
+    // the outputs of this thread: two rows of two neighbours (8-byte accesses
+    // at any 4-byte address), the residual on its way while the others arrive
+    const int oc = blockIdx.x * 16 * OB + row;
+    const int oy = 2 * ty, ox = 2 * tx;
+    const bool live = tile_ok && oc < M;
+    const long long base = live ? ((long long)img * M + oc) * HW + (long long)oy * W + ox : 0;
+    const int row1 = oy + 1 < H ? W : 0;  // the second row, or the first again
+    float rv[4] = {0.f, 0.f, 0.f, 0.f};
+    if (res && live) {
+        const float *src = res + base;
+        if (in2) {
+            const f32x2u a = *reinterpret_cast<const f32x2u *>(src), b = *reinterpret_cast<const f32x2u *>(src + row1);
+            rv[0] = a[0], rv[1] = a[1], rv[2] = b[0], rv[3] = b[1];
+        } else {
+            rv[0] = src[0], rv[2] = src[row1];
+        }
     }
     __syncthreads();
-    const int oc = ob * 16 + row;
-    if (!tile_ok || oc >= M) return;
+    if (!live) return;
     float m[16];
 #pragma unroll
-    for (int comp = 0; comp < 16; comp++) m[comp] = vs[0][comp * 256 + row * 16 + tl];
+    for (int comp = 0; comp < 16; comp++) m[comp] = ms[comp * MPLANE + tid];
     float t[8];
 #pragma unroll
     for (int j = 0; j < 4; j++) {  // A^T M
@@ -222,17 +285,18 @@ __global__ __launch_bounds__(256) void wino_f23_kernel(osh_conv_params p, const 
     o[1] = t[1] - t[2] - t[3] + b;
     o[2] = t[4] + t[5] + t[6] + b;
     o[3] = t[5] - t[6] - t[7] + b;
-    const int oy = 2 * ty, ox = 2 * tx;
-    const long long base = ((long long)img * M + oc) * H * W;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        const int yy = oy + (e >> 1), xx = ox + (e & 1);
-        if (yy < H && xx < W) {
-            const long long at = base + (long long)yy * W + xx;
-            float v = activate<ACT>(o[e]);
-            if (res) v = v + res[at];
-            y[at] = v;
-        }
+        o[e] = activate<ACT>(o[e]);
+        if (res) o[e] = o[e] + rv[e];
+    }
+    float *dst = y + base;
+    if (in2) {
+        *reinterpret_cast<f32x2u *>(dst) = f32x2u{o[0], o[1]};
+        if (row1) *reinterpret_cast<f32x2u *>(dst + row1) = f32x2u{o[2], o[3]};
+    } else {
+        dst[0] = o[0];
+        if (row1) dst[row1] = o[2];
     }
 }
 

@@ -307,6 +307,12 @@ WINOGRAD_CASES = [
     ("odd_24to40_33x45", (1, 24, 33, 45), (40, 24, 3, 3), "Silu", True),
     ("min_8to8_6x6", (1, 8, 6, 6), (8, 8, 3, 3), None, False),
     ("partial_40to24_7x9_no_bias", (1, 40, 7, 9), (24, 40, 3, 3), "Silu", False),
+    # two output blocks a workgroup: a half last block, a partial last chunk, odd maps; one partial
+    # chunk; workgroups over several images
+    ("two_blocks_40to72_31x33", (5, 40, 31, 33), (72, 40, 3, 3), "Silu", True),
+    ("two_blocks_8to48_30x30", (16, 8, 30, 30), (48, 8, 3, 3), None, True),
+    ("two_blocks_16to100_14x14", (24, 16, 14, 14), (100, 16, 3, 3), "Relu", False),
+    ("one_block_32to16_20x21", (8, 32, 20, 21), (16, 32, 3, 3), None, True),
 ]
 
 
