@@ -23,8 +23,10 @@
 //   1x1 / stride 1 / pad 0, C % 16 == 0 -> the LDS-tile kernel with one tap, or the GEMM tile,
 //                                          tuned per shape (the GEMM chain over ic)
 //   other 1x1 / stride 1 / pad 0        -> MFMA GEMM over NCHW (W[M,C] x X[C,H*W])
-//   everything else                     -> MFMA implicit GEMM with an im2col gather, k in the
-//                                          im2col order ic -> ky -> kx (ConvKernels.cs, PackedConv.cs)
+//   everything else                     -> gen_conv_kernel (osh_conv_gen.h): MFMA over an input patch
+//                                          in LDS, or, where no patch fits, the implicit GEMM with an
+//                                          im2col gather; k in the im2col order ic -> ky -> kx
+//                                          (ConvKernels.cs, PackedConv.cs)
 //
 // osh_config "winograd" = 0 leaves Winograd out (those shapes take the im2col
 // chain), 2 puts it ahead of the NCHWc kernels (the reference's choice on a
@@ -44,6 +46,7 @@
 
 #include "osh_conv16.h"
 #include "osh_conv16s.h"
+#include "osh_conv_gen.h"
 #include "osh_conv_pair.h"
 #include "osh_igemm.h"
 #include "osh_launch.h"
@@ -488,7 +491,7 @@ static bool nchwc_gate(const osh_conv_params *p) {
 }
 
 enum ConvAlgo { ALGO_DEPTHWISE = 0, ALGO_POINTWISE = 1, ALGO_IM2COL = 3, ALGO_FIRST = 6, ALGO_CONV16 = 7, ALGO_PW16 = 8,
-                ALGO_WINOGRAD = 9, ALGO_CONV16I = 10 };
+                ALGO_WINOGRAD = 9, ALGO_CONV16I = 10, ALGO_GEN = 11 };
 
 static bool is_pointwise(const osh_conv_params *p) {
     return p->kh == 1 && p->kw == 1 && p->sh == 1 && p->sw == 1 && p->pt == 0 && p->pl == 0 && p->oh == p->h &&
@@ -509,9 +512,9 @@ static ConvAlgo select_algo(const osh_conv_params *p) {
     if (first_conv_eligible(p)) return ALGO_FIRST;
     if (pointwise_variant() != -2 && pw16_eligible(p)) return ALGO_PW16;
     if (is_pointwise(p)) return ALGO_POINTWISE;
-    // the implicit-im2col GEMM: k in the order ic -> ky -> kx, the
-    // reference's im2col and panel chain
-    return ALGO_IM2COL;
+    // over an LDS patch where one fits, else the gathering GEMM: k in the
+    // order ic -> ky -> kx, the reference's im2col and panel chain
+    return gen_conv_eligible(p) ? ALGO_GEN : ALGO_IM2COL;
 }
 
 // ------------------------------------------------------------ conv16 tuning
@@ -888,6 +891,7 @@ OSH_API osh_status osh_conv_packed_weight_bytes(const osh_conv_params *p, size_t
     case ALGO_CONV16:
     case ALGO_CONV16I: *bytes = conv16_packed_bytes(p); break;
     case ALGO_WINOGRAD: *bytes = winograd_packed_bytes(p); break;
+    case ALGO_GEN: *bytes = gen_conv_packed_bytes(p); break;
     case ALGO_PW16: *bytes = conv16_packed_bytes(p) + oihw; break;  // LDS-tile layout, then the raw GEMM operand
     default: *bytes = oihw;
     }
@@ -923,6 +927,7 @@ static osh_status pack_weights(const osh_conv_params *p, const float *d_w, void 
     osh_status st = OSH_OK;
     if (select_algo(p) == ALGO_CONV16) return conv16_pack(p, d_w, d_packed, to_stream(s));
     if (select_algo(p) == ALGO_WINOGRAD) return winograd_pack(p, d_w, d_packed, to_stream(s));
+    if (select_algo(p) == ALGO_GEN) return gen_conv_pack(p, d_w, d_packed, to_stream(s));
     if (select_algo(p) == ALGO_CONV16I) return conv16_pack(p, d_w, d_packed, to_stream(s), true);
     if (select_algo(p) == ALGO_PW16) {
         st = conv16_pack(p, d_w, d_packed, to_stream(s));
@@ -1101,6 +1106,8 @@ static osh_status conv2d(const osh_conv_params *p, const float *d_x, const void 
             },
             stream);
     }
+    case ALGO_GEN:
+        return gen_conv_launch(p, d_x, w, d_bias, d_res, act, d_y, stream);
     case ALGO_POINTWISE:
     case ALGO_IM2COL:
         return igemm_conv(p, d_x, w, d_bias, d_res, act, d_y, stream,

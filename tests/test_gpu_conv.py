@@ -968,3 +968,45 @@ def test_depthwise_group_in_strips(cuda):
         torch.cuda.synchronize()
         for y, e in zip(ys, want):
             assert torch.equal(y, e)
+
+
+GEN_CASES = [
+    # (x shape, w shape, attrs, residual): convs only the general kernel takes
+    ((1, 3, 61, 67), (64, 3, 7, 7), dict(strides=[2, 2], pads=[3, 3, 3, 3]), False),  # K = 147, a plane of zeros
+    ((3, 3, 40, 33), (24, 3, 5, 5), dict(strides=[2, 2], pads=[2, 2, 2, 2]), True),   # two blocks, batch
+    ((1, 40, 37, 41), (24, 40, 3, 3), dict(strides=[2, 2], pads=[1, 1, 1, 1]), False),  # K = 360: a half last chunk
+    ((1, 200, 13, 11), (72, 200, 3, 3), dict(strides=[2, 2], pads=[1, 1, 1, 1]), True),  # many chunks, five blocks
+    ((2, 24, 15, 14), (32, 6, 3, 3), dict(group=4, pads=[1, 1, 1, 1]), False),        # groups of 8 outputs
+    ((1, 48, 21, 23), (80, 48, 1, 1), dict(strides=[2, 2]), False),                   # 1x1 stride 2
+    ((1, 20, 18, 20), (17, 20, 2, 2), dict(strides=[2, 2]), False),                   # even kernel, one row past a block
+    ((1, 6, 19, 30), (9, 6, 3, 5), dict(strides=[2, 1], pads=[1, 2, 1, 2], dilations=[1, 3]), True),
+    ((1, 33, 9, 1), (16, 33, 3, 1), dict(pads=[1, 0, 1, 0]), False),                  # one output column
+    ((1, 7, 1, 50), (40, 7, 1, 7), dict(pads=[0, 3, 0, 3]), False),                   # one output row
+    ((4, 8, 100, 96), (144, 8, 3, 3), dict(pads=[1, 1, 1, 1]), False),                # nine blocks, a large grid
+    ((2, 56, 100, 100), (48, 56, 3, 3), dict(pads=[1, 1, 1, 1]), True),               # three blocks of a large conv
+    ((1, 2, 90, 100), (3, 2, 5, 5), dict(dilations=[20, 20]), False),                 # no patch fits: the gathering GEMM
+]
+
+
+@pytest.mark.parametrize("xs,ws,attrs,residual", GEN_CASES, ids=[f"{c[0]}_{c[1]}" for c in GEN_CASES])
+def test_general_conv_is_the_im2col_chain(cuda, oracle, xs, ws, attrs, residual):
+    """The general kernel's tiles, chunks and blocks at their edges: bit for bit
+    the im2col chain from the bias; a NaN in the input reaches only its windows."""
+    from onnxsharp_amd import native as N
+    from onnxsharp_amd.layers import ConvLayer
+    print(f"general conv x={xs} w={ws} {attrs}", flush=True)
+    seed = sum(xs) * 19 + sum(ws)
+    x = synth.uniform(seed, xs, -1, 1)
+    x.reshape(-1)[x.size // 3] = np.nan
+    w = synth.normal(seed + 1, ws, 0, 0.1)
+    b = synth.normal(seed + 2, (ws[0],), 0, 0.01)
+    layer = ConvLayer(fused_activation="Relu", **attrs)
+    p = layer.resolve(xs, ws)
+    r = synth.normal(seed + 3, (p.n, p.m, p.oh, p.ow), 0, 1) if residual else None
+    N.kernel_log(True)
+    y = layer.forward(_t(x, cuda), _t(w, cuda), _t(b, cuda), residual=None if r is None else _t(r, cuda)).cpu().numpy()
+    assert any(("igemm" if max(p.dh, p.dw) == 20 else "gen_conv") in k for k in N.kernel_log(True))
+    ref = oracle_conv(oracle, x, w, b, p, "Relu", order=oracle.ORDER_IM2COL)
+    if r is not None:
+        ref = ref + r
+    assert np.array_equal(y, ref, equal_nan=True), f"max |d| {np.nanmax(np.abs(y - ref)):.3e}"
