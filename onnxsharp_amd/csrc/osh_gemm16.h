@@ -29,9 +29,11 @@
 //     of B[k0 + 4s + g][col .. col + BV - 1], col = 16*BV*tn + BV*j; component
 //     q feeds output block q of the tile, whose column j stands for col + q, so
 //     a lane stores BV adjacent columns at once.
-// k offsets live in scalar registers.  Rows past M and columns past N are
-// clamped for loads and never stored; the K tail (K % KC) is loaded with
-// guarded loads and zero-filled, and a zero product leaves the chain unchanged.
+// k offsets live in scalar registers.  Loads go through buffer descriptors, so
+// 4-byte alignment is enough for every width and no load sits under a
+// condition: rows past M are clamped, columns past N computed and never stored,
+// the K tail (K % KC) zero-filled, and a zero product leaves the chain
+// unchanged.
 #pragma once
 
 #include "osh_common.h"
@@ -85,7 +87,60 @@ struct G16B {
     G16Vec<BV> v[KC / 4][TN];  // one BV-wide load per k4 step and column block
 };
 
-template <int TM, int TN, int BV, int KC, int ACT>
+// Epilogue of a (16 * TM) x (16 * BV * TN) wave tile: column scale (fmaf),
+// activation, residual, BV-wide accesses (any 4-byte address will do).  RAG
+// (N % BV != 0) stores the columns of a vector that crosses N one by one; it is
+// a template parameter because that code beside the other, reached or not, cost
+// the compiler's schedule of the main loop (4096 x 1024 x 4096 247 -> 321 us).
+template <int TM, int TN, int BV, int ACT, bool RAG>
+__device__ __forceinline__ void g16_store(const IgemmArgs &p, const f32x4 (&acc)[TM][TN * BV], int m0, int n0, int j,
+                                          int g, int zo, int zi) {
+    const int N = p.N;
+    float *C = p.C + zo * p.strideC + zi * p.strideC_in;
+    const float *R = p.res ? p.res + zo * p.strideC + zi * p.strideC_in : nullptr;
+#pragma unroll
+    for (int tm = 0; tm < TM; tm++)
+#pragma unroll
+        for (int tn = 0; tn < TN; tn++) {
+            const int col = n0 + 16 * BV * tn + BV * j;
+            if (col >= N) continue;
+            float cs[BV], cb[BV];
+#pragma unroll
+            for (int q = 0; q < BV; q++) {
+                const int cq = RAG ? min(col + q, N - 1) : col + q;
+                cs[q] = p.col_scale ? p.col_scale[cq] : 0.f;
+                cb[q] = (p.col_scale && p.col_bias) ? p.col_bias[cq] : 0.f;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int row = m0 + 16 * tm + 4 * g + r;
+                if (row >= p.M) continue;
+                float o[BV];
+#pragma unroll
+                for (int q = 0; q < BV; q++) {
+                    float v = acc[tm][tn * BV + q][r];
+                    if (p.col_scale) v = __builtin_fmaf(v, cs[q], cb[q]);
+                    o[q] = activate<ACT>(v);
+                }
+                const long long at = (long long)row * p.ldc + col;
+                if (!RAG || col + BV <= N) {
+                    if (R) {
+                        float t[BV];
+                        __builtin_memcpy(t, R + at, sizeof(t));
+#pragma unroll
+                        for (int q = 0; q < BV; q++) o[q] += t[q];
+                    }
+                    __builtin_memcpy(C + at, o, sizeof(o));
+                } else {
+#pragma unroll
+                    for (int q = 0; q < BV; q++)
+                        if (col + q < N) C[at + q] = R ? o[q] + R[at + q] : o[q];
+                }
+            }
+        }
+}
+
+template <int TM, int TN, int BV, int KC, int ACT, bool RAG>
 __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
     constexpr int STEPS = KC / 4;
     constexpr int AU = KC / 16;  // A float4 slots per lane per 16-row block
@@ -107,8 +162,6 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
     const int zo = z / p.zdiv, zi = z % p.zdiv;
     const float *__restrict__ A = p.A + zo * p.strideA + zi * p.strideA_in;
     const float *__restrict__ B = p.B + zo * p.strideB + zi * p.strideB_in;
-    float *__restrict__ C = p.C + zo * p.strideC + zi * p.strideC_in;
-    const float *__restrict__ R = p.res ? p.res + zo * p.strideC + zi * p.strideC_in : nullptr;
     const float *__restrict__ row_bias = p.row_bias ? p.row_bias + zi * p.bias_stride : nullptr;
     const int M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb;
     const int bytes_a = (int)(((long long)(M - 1) * lda + K) * 4);
@@ -129,7 +182,13 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
     const int lr = j * 16 + g * 4;  // lane (j, g) reads [tm][kg][j][g][0..3]
     int vob[TN];
 #pragma unroll
-    for (int tn = 0; tn < TN; tn++) vob[tn] = (g * ldb + min(n0 + 16 * BV * tn + BV * j, N - BV)) * 4;
+    for (int tn = 0; tn < TN; tn++) {
+        // a vector that starts past N reads column 0 instead; one that
+        // crosses N reads on into the next row; neither part is stored
+        const int col = n0 + 16 * BV * tn + BV * j;
+                vob[tn] = (g * ldb + (col < N ? col : 0)) * 4;
+
+    }
 
     f32x4 acc[TM][TN * BV];
 #pragma unroll
@@ -162,6 +221,15 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
                 R.v[tm][u] = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
                                          __uint_as_float(v[3]));
             }
+    };
+    // Rows past K (the tail chunk) are left to the range check, which compares
+    // the vector offset alone with the operand's size: their k goes there.
+    auto load_b_tail = [&](G16B<TN, BV, KC> &R, int c) {
+        __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, (short)0, bytes_b, 0x00020000);
+#pragma unroll
+        for (int s = 0; s < STEPS; s++)
+#pragma unroll
+            for (int tn = 0; tn < TN; tn++) R.v[s][tn] = g16_load_b<BV>(rb, vob[tn] + (c * KC + 4 * s) * ldb * 4, 0);
     };
     auto load_b = [&](G16B<TN, BV, KC> &R, int c) {
         __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, (short)0, bytes_b, 0x00020000);
@@ -258,87 +326,32 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
         if (c < nfull) compute(av0, rb0);
     }
     if (K % KC) {
-        // tail chunk: k >= K loads as zero; staged through buffer 0 (every
-        // earlier read of it has completed: LDS accesses of a wave are in order)
+        // tail chunk: B's rows past K lie past its descriptor and read as zero,
+        // A's k past K (the next row's) are zeroed; staged through buffer 0
+        // (every earlier read of it has completed: LDS accesses of a wave are
+        // in order)
         G16A<TM, KC> ra;
         G16B<TN, BV, KC> rb;
         G16AV<TM, KC> av;
-        const int k0 = nfull * KC;
+        load_a(ra, nfull);
+        load_b_tail(rb, nfull);
 #pragma unroll
         for (int tm = 0; tm < TM; tm++)
 #pragma unroll
             for (int u = 0; u < AU; u++) {
-                const int e = lane + 64 * u, r = e / KQ, kq = e % KQ;
-                const float *src = A + (long long)min(m0 + 16 * tm + r, M - 1) * lda;
-                float t4[4];
-#pragma unroll
-                for (int c2 = 0; c2 < 4; c2++) {
-                    const int k = k0 + 4 * kq + c2;
-                    t4[c2] = k < K ? src[k] : 0.f;
-                }
-                ra.v[tm][u] = make_float4(t4[0], t4[1], t4[2], t4[3]);
+                const int k = nfull * KC + 4 * ((lane + 64 * u) % KQ);
+                float4 &v = ra.v[tm][u];
+                v.x = k + 0 < K ? v.x : 0.f;
+                v.y = k + 1 < K ? v.y : 0.f;
+                v.z = k + 2 < K ? v.z : 0.f;
+                v.w = k + 3 < K ? v.w : 0.f;
             }
-#pragma unroll
-        for (int s = 0; s < STEPS; s++) {
-            const int k = k0 + 4 * s + g;
-#pragma unroll
-            for (int tn = 0; tn < TN; tn++) {
-                const int col = min(n0 + 16 * BV * tn + BV * j, N - BV);
-#pragma unroll
-                for (int q = 0; q < BV; q++) rb.v[s][tn].v[q] = k < K ? B[(long long)k * ldb + col + q] : 0.f;
-            }
-        }
         stage_a(ra, 0);
         read_a(av, 0);
         compute(av, rb);
     }
 
-    // ---- epilogue: column scale (fmaf), activation, BV-wide stores
-#pragma unroll
-    for (int tm = 0; tm < TM; tm++)
-#pragma unroll
-        for (int tn = 0; tn < TN; tn++) {
-            const int col = n0 + 16 * BV * tn + BV * j;
-            if (col >= N) continue;
-            float cs[BV], cb[BV];
-#pragma unroll
-            for (int q = 0; q < BV; q++) {
-                cs[q] = p.col_scale ? p.col_scale[col + q] : 0.f;
-                cb[q] = (p.col_scale && p.col_bias) ? p.col_bias[col + q] : 0.f;
-            }
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = m0 + 16 * tm + 4 * g + r;
-                if (row >= M) continue;
-                float o[BV];
-#pragma unroll
-                for (int q = 0; q < BV; q++) {
-                    float v = acc[tm][tn * BV + q][r];
-                    if (p.col_scale) v = __builtin_fmaf(v, cs[q], cb[q]);
-                    o[q] = activate<ACT>(v);
-                }
-                if (R) {  // residual: same layout as C, BV-wide loads
-                    const float *src = R + (long long)row * p.ldc + col;
-                    if constexpr (BV == 4) {
-                        const float4 t = *reinterpret_cast<const float4 *>(src);
-                        o[0] += t.x, o[1] += t.y, o[2] += t.z, o[3] += t.w;
-                    } else if constexpr (BV == 2) {
-                        const float2 t = *reinterpret_cast<const float2 *>(src);
-                        o[0] += t.x, o[1] += t.y;
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < BV; q++) o[q] += src[q];
-                    }
-                }
-                float *dst = C + (long long)row * p.ldc + col;
-                if constexpr (BV == 4) *reinterpret_cast<float4 *>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-                else if constexpr (BV == 2) *reinterpret_cast<float2 *>(dst) = make_float2(o[0], o[1]);
-                else {
-#pragma unroll
-                    for (int q = 0; q < BV; q++) dst[q] = o[q];
-                }
-            }
-        }
+    g16_store<TM, TN, BV, ACT, RAG>(p, acc, m0, n0, j, g, zo, zi);
 }
 
 }  // namespace osh

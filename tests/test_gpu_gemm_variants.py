@@ -72,6 +72,37 @@ def test_gemm_variants_column_bias(cuda, oracle, variant_reset, m, k, n, lpad, c
         assert np.array_equal(y, ref), f"variant {v} gemm {m}x{k}x{n}: not bit-identical"
 
 
+@pytest.mark.parametrize("m,k,n,off", [(1, 1, 1, 1), (17, 31, 2, 1), (16, 33, 47, 3), (33, 65, 49, 2), (35, 97, 131, 1)])
+def test_gemm_variants_ragged_rows(cuda, oracle, variant_reset, m, k, n, off):
+    """Odd rows at odd addresses: one chain of fmafs, bit for bit, and nothing
+    of what surrounds the operands (NaN here: a leading dimension's padding,
+    the floats before and after) reaches the result."""
+    import torch
+    from onnxsharp_amd import native as N
+    a = synth.uniform(m * 11 + k, (m, k), -1, 1)
+    b = synth.uniform(n * 3 + k, (k, n), -1, 1)
+    res = synth.uniform(m + n + k, (n,), -1, 1)
+    lda, ldb, ldc = k + off, n + off, n + 1
+
+    def held(x, ld):  # NaN around and between the rows
+        buf = np.full((off + x.shape[0] * ld + 80,), np.nan, np.float32)
+        buf[off:off + x.shape[0] * ld].reshape(-1, ld)[:, :x.shape[1]] = x
+        return _t(buf, cuda)
+
+    da, db, bias = held(a, lda), held(b, ldb), _t(res, cuda)
+    at = lambda t, o: C.c_void_p(t.data_ptr() + 4 * o)
+    ref = oracle.gemm_f32(a, b, col_bias=res)
+    for v in _variants()[1:] + [-1]:
+        print(f"gemm variant {v}: m={m} k={k} n={n} offset={off}", flush=True)
+        N.call("osh_config_set", b"gemm_variant", v)
+        dc = torch.full((off + m * ldc,), 7.0, dtype=torch.float32, device=cuda)
+        N.call("osh_gemm_f32", m, n, k, at(da, off), lda, at(db, off), ldb, at(bias, 0), None, None, 0, at(dc, off),
+               ldc, C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        y = dc.cpu().numpy()
+        assert (y[:off] == 7.0).all() and (y[off:].reshape(m, ldc)[:, n:] == 7.0).all(), "wrote past n"
+        assert np.array_equal(y[off:].reshape(m, ldc)[:, :n], ref), f"variant {v}: not bit-identical"
+
+
 def test_gemm_variants_row_bias_silu_and_column_scale(cuda, oracle, variant_reset):
     from onnxsharp_amd import native as N
     m, k, n = 128, 256, 640
