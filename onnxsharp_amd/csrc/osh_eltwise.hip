@@ -300,6 +300,80 @@ __global__ __launch_bounds__(256) void softmax_kernel(long long rows, int cols, 
         for (int c = lane; c < cols; c += 64) yr[c] = buf[c] * inv;
 }
 
+// Rows of at most 64 * NE columns, two a wave: the values stay in registers
+// from the load to the store (loads clamp to the last column, which leaves the
+// max alone, so none sits under a condition), and the rows' lane sums run side
+// by side: lane 8r + k adds row r's columns 8j + k in order of j, eight LDS
+// reads ahead.  What bounds a launch is latency, not the 8 bytes an element, and
+// softmax_kernel's one row a wave had a chain of cols / 8 LDS reads on eight
+// lanes.  3084 x 257: 5.5 -> 4.1 us, 6120 x 510: 11.3 -> 7.2, 186 x 62: 3.1 ->
+// 2.6 (one row a wave 4.1 / 7.9 / 2.5, four 4.8 / 8.0 / 3.0).
+constexpr int SOFTMAX_ROWS = 2;
+
+template <int NE>
+__global__ __launch_bounds__(256) void softmax_rows_kernel(long long rows, int cols, float scale,
+                                                           const float *__restrict__ x, float *__restrict__ y) {
+    constexpr int R = SOFTMAX_ROWS;
+    constexpr int PITCH = 64 * NE + 8;  // rows 8 banks apart: the lane sums read 32 different ones
+    __shared__ float srow[4 * R * PITCH];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const long long row0 = ((long long)blockIdx.x * 4 + wave) * R;
+    float *buf = srow + wave * (R * PITCH);
+    if (row0 >= rows) return;  // whole wave; the kernel has no barriers
+    float e[R][NE], m[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const float *xr = x + (row0 + r < rows ? row0 + r : rows - 1) * cols;
+#pragma unroll
+        for (int i = 0; i < NE; i++) e[r][i] = xr[min(lane + 64 * i, cols - 1)];
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        m[r] = -__builtin_inff();
+#pragma unroll
+        for (int i = 0; i < NE; i++) m[r] = __builtin_fmaxf(m[r], e[r][i] * scale);
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) m[r] = wave_max_f(m[r]);
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            e[r][i] = exp_ref(e[r][i] * scale - m[r]);
+            buf[r * PITCH + lane + 64 * i] = e[r][i];  // past cols: never summed
+        }
+    // a wave's LDS accesses complete in order: no barrier
+    const int rl = (lane >> 3) & (R - 1), k = lane & 7;  // lanes past 8 R repeat a row
+    const float *br = buf + rl * PITCH;
+    const int nj = cols >> 3;
+    float part = 0.0f;
+    for (int j0 = 0; j0 < nj; j0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = br[min(8 * (j0 + j), 64 * NE - 8) + k];
+#pragma unroll
+        for (int j = 0; j < 8; j++) part = j0 + j < nj ? part + v[j] : part;
+    }
+    float tail[7], sum = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 7; t++) tail[t] = br[min(8 * nj + t, 64 * NE - 1)];
+#pragma unroll
+    for (int q = 0; q < 8; q++) sum = sum + __shfl(part, (lane & ~7) + q);
+#pragma unroll
+    for (int t = 0; t < 7; t++) sum = 8 * nj + t < cols ? sum + tail[t] : sum;
+    const float inv = 1.0f / sum;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const float ir = __shfl(inv, 8 * r);
+        if (row0 + r < rows) {
+            float *yr = y + (row0 + r) * cols;
+#pragma unroll
+            for (int i = 0; i < NE; i++)
+                if (lane + 64 * i < cols) yr[lane + 64 * i] = e[r][i] * ir;
+        }
+    }
+}
+
 static unsigned grid_for(long long n, long long per_block, long long cap) {
     long long b = (n + per_block - 1) / per_block;
     if (b < 1) b = 1;
@@ -427,6 +501,18 @@ OSH_API osh_status osh_softmax_f32(int64_t rows, int cols, float scale, const fl
     if (rows == 0 || cols == 0) return OSH_OK;
     if (!d_x || !d_y) return fail(OSH_E_INVALID, "Softmax: NULL pointer");
     if (d_x == d_y) return fail(OSH_E_INVALID, "Softmax: in-place is not supported");
+    // up to 512 columns the row fits eight registers a lane
+#define OSH_SOFTMAX_ROWS(NE)                                                                                          \
+    case NE:                                                                                                          \
+        OSH_LAUNCH(softmax_rows_kernel<NE>, dim3(grid_for(rows, 4 * SOFTMAX_ROWS, 0x7fffffff)), dim3(256), 0,         \
+                   to_stream(s), (long long)rows, cols, scale, d_x, d_y);                                             \
+        OSH_LAUNCH_CHECK("softmax_rows_kernel");                                                                      \
+        return OSH_OK;
+    switch ((cols + 63) / 64) {
+        OSH_SOFTMAX_ROWS(1) OSH_SOFTMAX_ROWS(2) OSH_SOFTMAX_ROWS(3) OSH_SOFTMAX_ROWS(4)
+        OSH_SOFTMAX_ROWS(5) OSH_SOFTMAX_ROWS(6) OSH_SOFTMAX_ROWS(7) OSH_SOFTMAX_ROWS(8)
+    }
+#undef OSH_SOFTMAX_ROWS
     if (cols <= SOFTMAX_LDS_COLS)
         OSH_LAUNCH(softmax_kernel<true>, dim3(grid_for(rows, 4, 0x7fffffff)), dim3(256),
                            (size_t)4 * cols * sizeof(float), to_stream(s), (long long)rows, cols, scale, d_x, d_y);

@@ -138,6 +138,24 @@ def test_transpose_last_two_axes(cuda, batch, rows, cols):
     assert np.array_equal(y.cpu().numpy(), x.transpose(0, 2, 1))
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (2, 7), (3, 64), (5, 65), (17, 127), (9, 257), (8, 511), (7, 512),
+                                       (7, 513)])
+def test_softmax_row_widths(cuda, oracle, rows, cols):
+    # every register count of the row kernel, a last wave with one row, and
+    # masked columns (the type's lowest value): the oracle's bits
+    import torch
+    from onnxsharp_amd import native as N
+    x = synth.normal(970 + cols, (rows, cols), 0, 4)
+    x[rows // 2, 1:] = np.finfo(np.float32).min
+    dx = _dev(x, cuda)
+    y = torch.full((rows + 1, cols), 7.0, device=cuda)
+    N.call("osh_softmax_f32", rows, cols, C.c_float(0.125), _p(dx), _p(y), None)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.array_equal(got[:rows], oracle.softmax(x, 0.125)), f"softmax {rows}x{cols}"
+    assert (got[rows] == 7.0).all(), "wrote past the last row"
+
+
 @pytest.mark.parametrize("rows,cols,scale", [(800, 400, 32 ** -0.5), (7, 1000, 1.0), (3, 5, 10.0), (9, 13, 0.5),
                                               (33, 8, 1.0)])
 def test_softmax_is_the_reference_row_order(cuda, oracle, rows, cols, scale):
