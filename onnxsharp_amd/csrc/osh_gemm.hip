@@ -51,14 +51,28 @@ static bool g16_fits(const IgemmArgs &a) {
     return a.K >= 1 && ((a.M - 1LL) * a.lda + kmax) * 4 < (1LL << 31) && (kmax * a.ldb + a.N + 64) * 4 < (1LL << 31);
 }
 
-// Predicted cost: rounds of waves over the SIMDs times the MFMAs of one wave
-// tile, inflated by the operand traffic per MFMA (TN B loads and about TM/2
-// A loads feed TM*TN*BV MFMAs per k4 step).
+// Predicted time of a wave tile, in cycles up to a common factor.  A wave's
+// chunk takes its MFMAs or, where those are fewer, one trip to memory (loads are
+// one chunk ahead): 600 in L2, 715 past it, for 32 k; 64-k chunks pay only where
+// the operands (A and B together) exceed the 4 MB of an XCD's L2, since their 16
+// MFMAs a block are no shorter a chain.  Waves beyond one a SIMD
+// add their MFMAs, and part of their prologue and epilogue, which overlap.
+// Workgroups of four waves fill the chip by fours, so slots count, not tiles
+// (of fewer row tiles the idle waves leave at once).
+// Fitted to 178 products (m 1-4096, k 32-4096, n 32-8192): on average 1.4% above
+// the best tile of each, the former rule (rounds of waves times MFMAs, inflated
+// by loads an MFMA) 6.8% and up to 57% (208 x 2952 x 1226 66 -> 42 us, 16 x 3566
+// x 1223 43 -> 28, 820 x 384 x 1760 25 -> 17).
 static double g16_cost(const IgemmArgs &a, int zcount, const G16Variant &v, int cus) {
-    const long long waves = (long long)ceil_div(a.M, 16 * v.tm) * ceil_div(a.N, 16 * v.bv * v.tn) * zcount;
-    const long long rounds = (waves + 4LL * cus - 1) / (4LL * cus);
+    const int tiles_m = ceil_div(a.M, 16 * v.tm), waves = std::min(tiles_m, 4);
+    const double slots = (double)ceil_div(tiles_m, waves) * waves * ceil_div(a.N, 16 * v.bv * v.tn) * zcount;
     const double u = (double)v.tm * v.tn * v.bv;
-    return rounds * u * ceil_div(a.K, 4) * (1.0 + 0.5 * (v.tn + 0.5 * v.tm) / u);
+    const bool far = 4.0 * zcount * ((double)a.M * a.K + (double)a.K * a.N) > 4.2e6;  // an XCD's L2: 4 MB
+    const double chunks = ceil_div(a.K, v.kc), mfma = v.kc / 4 * 22.0 * u;
+    const double trip = v.kc == 32 ? (far ? 715 : 600) : (far ? 1270 + 60 * u : 4000);
+    const double per_simd = slots / (4.0 * cus);
+    const double more = std::max(0.0, 0.2 * std::ceil(per_simd) + 0.8 * per_simd - 1.0);
+    return 3800 + 450 * u + chunks * std::max(trip, mfma + 60) + more * (1.15 * chunks * mfma + 270 * u);
 }
 
 template <int TM, int TN, int BV, int KC>
@@ -68,8 +82,8 @@ static osh_status g16_launch(const IgemmArgs &a, int zcount, int act, hipStream_
     if (blocks > 0x7fffffffLL) return fail(OSH_E_UNSUPPORTED, "GEMM grid too large");
     dim3 grid((unsigned)blocks, zcount);
     if (a.N % BV) {
-        OSH_DISPATCH_ACT(act, ACT, OSH_LAUNCH((gemm16_kernel<TM, TN, BV, KC, ACT, (BV > 1)>), grid, dim3(256), 0, st, a,
-                                              tiles_m));
+        OSH_DISPATCH_ACT(act, ACT, OSH_LAUNCH((gemm16_kernel<TM, TN, BV, KC, ACT, (BV > 1)>), grid, dim3(256), 0, st,
+                                              a, tiles_m));
     } else {
         OSH_DISPATCH_ACT(act, ACT,
                          OSH_LAUNCH((gemm16_kernel<TM, TN, BV, KC, ACT, false>), grid, dim3(256), 0, st, a, tiles_m));
