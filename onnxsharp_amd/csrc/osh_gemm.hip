@@ -54,12 +54,14 @@ static bool g16_fits(const IgemmArgs &a) {
 // Predicted time of a wave tile, in cycles up to a common factor.  A wave's
 // chunk takes its MFMAs or, where those are fewer, one trip to memory (loads are
 // one chunk ahead): 600 in L2, 715 past it, for 32 k; 64-k chunks pay only where
-// the operands (A and B together) exceed the 4 MB of an XCD's L2, since their 16
-// MFMAs a block are no shorter a chain.  Waves beyond one a SIMD
+// the operands (A and B together) are well past the 4 MB of an XCD's L2, since
+// their 16 MFMAs a block are no shorter a chain (6 MB: at 4.3 MB 64-k chunks cost
+// 62 x 1984 x 480 14.3 -> 16.7 us with both operands in L2, and gave 13 x 417 x
+// 2572 8.0 -> 7.0 without).  Waves beyond one a SIMD
 // add their MFMAs, and part of their prologue and epilogue, which overlap.
 // Workgroups of four waves fill the chip by fours, so slots count, not tiles
 // (of fewer row tiles the idle waves leave at once).
-// Fitted to 178 products (m 1-4096, k 32-4096, n 32-8192): on average 1.4% above
+// Fitted to 180 products (m 1-4096, k 32-4096, n 32-8192): on average 1.8% above
 // the best tile of each, the former rule (rounds of waves times MFMAs, inflated
 // by loads an MFMA) 6.8% and up to 57% (208 x 2952 x 1226 66 -> 42 us, 16 x 3566
 // x 1223 43 -> 28, 820 x 384 x 1760 25 -> 17).
@@ -67,7 +69,7 @@ static double g16_cost(const IgemmArgs &a, int zcount, const G16Variant &v, int 
     const int tiles_m = ceil_div(a.M, 16 * v.tm), waves = std::min(tiles_m, 4);
     const double slots = (double)ceil_div(tiles_m, waves) * waves * ceil_div(a.N, 16 * v.bv * v.tn) * zcount;
     const double u = (double)v.tm * v.tn * v.bv;
-    const bool far = 4.0 * zcount * ((double)a.M * a.K + (double)a.K * a.N) > 4.2e6;  // an XCD's L2: 4 MB
+    const bool far = 4.0 * zcount * ((double)a.M * a.K + (double)a.K * a.N) > 6e6;
     const double chunks = ceil_div(a.K, v.kc), mfma = v.kc / 4 * 22.0 * u;
     const double trip = v.kc == 32 ? (far ? 715 : 600) : (far ? 1270 + 60 * u : 4000);
     const double per_simd = slots / (4.0 * cus);

@@ -94,10 +94,8 @@ struct G16B {
 // the compiler's schedule of the main loop (4096 x 1024 x 4096 247 -> 321 us).
 template <int TM, int TN, int BV, int ACT, bool RAG>
 __device__ __forceinline__ void g16_store(const IgemmArgs &p, const f32x4 (&acc)[TM][TN * BV], int m0, int n0, int j,
-                                          int g, int zo, int zi) {
-    const int N = p.N;
-    float *C = p.C + zo * p.strideC + zi * p.strideC_in;
-    const float *R = p.res ? p.res + zo * p.strideC + zi * p.strideC_in : nullptr;
+                                          int g, float *__restrict__ C, const float *__restrict__ R) {
+    const int M = p.M, N = p.N;
 #pragma unroll
     for (int tm = 0; tm < TM; tm++)
 #pragma unroll
@@ -114,7 +112,7 @@ __device__ __forceinline__ void g16_store(const IgemmArgs &p, const f32x4 (&acc)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int row = m0 + 16 * tm + 4 * g + r;
-                if (row >= p.M) continue;
+                if (row >= M) continue;
                 float o[BV];
 #pragma unroll
                 for (int q = 0; q < BV; q++) {
@@ -162,6 +160,8 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
     const int zo = z / p.zdiv, zi = z % p.zdiv;
     const float *__restrict__ A = p.A + zo * p.strideA + zi * p.strideA_in;
     const float *__restrict__ B = p.B + zo * p.strideB + zi * p.strideB_in;
+    float *__restrict__ C = p.C + zo * p.strideC + zi * p.strideC_in;
+    const float *__restrict__ R = p.res ? p.res + zo * p.strideC + zi * p.strideC_in : nullptr;
     const float *__restrict__ row_bias = p.row_bias ? p.row_bias + zi * p.bias_stride : nullptr;
     const int M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb;
     const int bytes_a = (int)(((long long)(M - 1) * lda + K) * 4);
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
         compute(av, rb);
     }
 
-    g16_store<TM, TN, BV, ACT, RAG>(p, acc, m0, n0, j, g, zo, zi);
+    g16_store<TM, TN, BV, ACT, RAG>(p, acc, m0, n0, j, g, C, R);
 }
 
 }  // namespace osh
