@@ -29,14 +29,18 @@
 //     of B[k0 + 4s + g][col .. col + BV - 1], col = 16*BV*tn + BV*j; component
 //     q feeds output block q of the tile, whose column j stands for col + q, so
 //     a lane stores BV adjacent columns at once.
-// k offsets live in scalar registers.  Loads go through buffer descriptors, so
-// 4-byte alignment is enough for every width and no load sits under a
-// condition: rows past M are clamped, columns past N computed and never stored,
-// the K tail (K % KC) zero-filled, and a zero product leaves the chain
+// k offsets live in scalar registers, or in the vector offset where a load may
+// reach past its operand (osh_gemm16_addr.h).  Loads go through buffer
+// descriptors, so 4-byte alignment is enough for every width and no load sits
+// under a condition: rows past M are clamped, columns past N computed and never
+// stored, the K tail (K % KC) zero-filled, and a zero product leaves the chain
 // unchanged.
 #pragma once
 
+#include <type_traits>
+
 #include "osh_common.h"
+#include "osh_gemm16_addr.h"
 #include "osh_igemm.h"
 
 namespace osh {
@@ -164,8 +168,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
     const float *__restrict__ R = p.res ? p.res + zo * p.strideC + zi * p.strideC_in : nullptr;
     const float *__restrict__ row_bias = p.row_bias ? p.row_bias + zi * p.bias_stride : nullptr;
     const int M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb;
-    const int bytes_a = (int)(((long long)(M - 1) * lda + K) * 4);
-    const int bytes_b = (int)(((long long)(K - 1) * ldb + N) * 4);
+    const int bytes_a = g16_bytes_a(M, K, lda), bytes_b = g16_bytes_b(K, N, ldb);
     float *wl = lds + wave * G16Lds<TM, KC>::WAVE;
 
     // A slot e = lane + 64u of a 16-row block: row e / KQ, k = 4 * (e % KQ);
@@ -176,19 +179,13 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
 #pragma unroll
         for (int u = 0; u < AU; u++) {
             const int e = lane + 64 * u, r = e / KQ, kq = e % KQ;
-            voa[tm][u] = (min(m0 + 16 * tm + r, M - 1) * lda + 4 * kq) * 4;
+            voa[tm][u] = g16_lane_a(min(m0 + 16 * tm + r, M - 1), kq, lda);
             lw[tm][u] = ((tm * (KC / 16) + (kq >> 2)) * 16 + r) * 16 + (kq & 3);
         }
     const int lr = j * 16 + g * 4;  // lane (j, g) reads [tm][kg][j][g][0..3]
     int vob[TN];
 #pragma unroll
-    for (int tn = 0; tn < TN; tn++) {
-        // a vector that starts past N reads column 0 instead; one that
-        // crosses N reads on into the next row; neither part is stored
-        const int col = n0 + 16 * BV * tn + BV * j;
-                vob[tn] = (g * ldb + (col < N ? col : 0)) * 4;
-
-    }
+    for (int tn = 0; tn < TN; tn++) vob[tn] = g16_lane_b(g, n0 + 16 * BV * tn + BV * j, N, ldb);
 
     f32x4 acc[TM][TN * BV];
 #pragma unroll
@@ -210,34 +207,32 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
 
     const int nfull = K / KC;
 
-    // Full chunks only (k0 + KC <= K): unguarded loads, scalar k offsets.
-    auto load_a = [&](G16A<TM, KC> &R, int c) {
+    // Chunk c; `tail` (a type, so that the full chunks' loads stay as they are)
+    // for the one that K ends in.
+    auto load_a = [&](G16A<TM, KC> &R, int c, auto tail) {
         __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)A, (short)0, bytes_a, 0x00020000);
 #pragma unroll
         for (int tm = 0; tm < TM; tm++)
 #pragma unroll
             for (int u = 0; u < AU; u++) {
-                auto v = __builtin_amdgcn_raw_buffer_load_b128(ra, voa[tm][u], c * KC * 4, 0);
+                const G16Off o = g16_off_a<decltype(tail)::value>(voa[tm][u], c * KC);
+                auto v = __builtin_amdgcn_raw_buffer_load_b128(ra, o.vec, o.scalar, 0);
                 R.v[tm][u] = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
                                          __uint_as_float(v[3]));
             }
     };
-    // Rows past K (the tail chunk) are left to the range check, which compares
-    // the vector offset alone with the operand's size: their k goes there.
-    auto load_b_tail = [&](G16B<TN, BV, KC> &R, int c) {
+    auto load_b = [&](G16B<TN, BV, KC> &R, int c, auto tail) {
         __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, (short)0, bytes_b, 0x00020000);
 #pragma unroll
         for (int s = 0; s < STEPS; s++)
 #pragma unroll
-            for (int tn = 0; tn < TN; tn++) R.v[s][tn] = g16_load_b<BV>(rb, vob[tn] + (c * KC + 4 * s) * ldb * 4, 0);
+            for (int tn = 0; tn < TN; tn++) {
+                const G16Off o = g16_off_b<decltype(tail)::value, RAG>(vob[tn], c * KC + 4 * s, ldb);
+                R.v[s][tn] = g16_load_b<BV>(rb, o.vec, o.scalar);
+            }
     };
-    auto load_b = [&](G16B<TN, BV, KC> &R, int c) {
-        __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)B, (short)0, bytes_b, 0x00020000);
-#pragma unroll
-        for (int s = 0; s < STEPS; s++)
-#pragma unroll
-            for (int tn = 0; tn < TN; tn++) R.v[s][tn] = g16_load_b<BV>(rb, vob[tn], (c * KC + 4 * s) * ldb * 4);
-    };
+    constexpr std::false_type full{};
+    constexpr std::true_type tail{};
     auto stage_a = [&](const G16A<TM, KC> &R, int buf) {
         float *dst = wl + buf * CH;
 #pragma unroll
@@ -284,12 +279,12 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
         G16A<TM, KC> ra;
         G16B<TN, BV, KC> rb0, rb1;
         G16AV<TM, KC> av0, av1;
-        load_a(ra, 0);
-        load_b(rb0, 0);
+        load_a(ra, 0, full);
+        load_b(rb0, 0, full);
         stage_a(ra, 0);
-        load_a(ra, min(1, last));
+        load_a(ra, min(1, last), full);
         stage_a(ra, 1);
-        load_a(ra, min(2, last));
+        load_a(ra, min(2, last), full);
         read_a(av0, 0);
         int c = 0;
         // The loads and LDS traffic of a half-step are issued between its
@@ -299,13 +294,13 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
         constexpr int NMF = STEPS * TM * TN * BV;  // MFMAs per chunk
         constexpr int NGR = (NMF + 1) / 2;          // groups of two
         for (; c + 2 <= nfull; c += 2) {
-            load_b(rb1, c + 1);
+            load_b(rb1, c + 1, full);
             __builtin_amdgcn_sched_barrier(0);
             compute(av0, rb0);
             read_a(av1, 1);            // A(c+1), staged a chunk ago
             stage_a(ra, 0);            // A(c+2) into the buffer chunk c used
-            load_a(ra, min(c + 3, last));
-            load_b(rb0, min(c + 2, last));
+            load_a(ra, min(c + 3, last), full);
+            load_b(rb0, min(c + 2, last), full);
 #pragma unroll
             for (int i = 0; i < NGR; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);                  // two MFMAs
@@ -315,7 +310,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
             compute(av1, rb1);
             read_a(av0, 0);            // A(c+2)
             stage_a(ra, 1);            // A(c+3)
-            load_a(ra, min(c + 4, last));
+            load_a(ra, min(c + 4, last), full);
 #pragma unroll
             for (int i = 0; i < NGR; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
@@ -327,14 +322,14 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
     }
     if (K % KC) {
         // tail chunk: B's rows past K lie past its descriptor and read as zero,
-        // A's k past K (the next row's) are zeroed; staged through buffer 0
-        // (every earlier read of it has completed: LDS accesses of a wave are
-        // in order)
+        // A's k past K (the next row's, or nothing) are zeroed; staged through
+        // buffer 0 (every earlier read of it has completed: LDS accesses of a
+        // wave are in order)
         G16A<TM, KC> ra;
         G16B<TN, BV, KC> rb;
         G16AV<TM, KC> av;
-        load_a(ra, nfull);
-        load_b_tail(rb, nfull);
+        load_a(ra, nfull, tail);
+        load_b(rb, nfull, tail);
 #pragma unroll
         for (int tm = 0; tm < TM; tm++)
 #pragma unroll
