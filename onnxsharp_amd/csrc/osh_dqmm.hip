@@ -695,13 +695,17 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
 #pragma unroll
             for (int i = 0; i < DQF_KS; i++) dst[i * 256] = (int)quantize4(x[i], inv, zpf, 0xfu, sum, nan);
         } else {
-            // k % 4 == 0: a quad is all inside its row or not there at all (its
-            // loads then gave zeros: no NaN), so one select masks it
+            // k % 4 == 0: a quad is all inside its row or not there at all, so
+            // one select masks it, and one its NaN flag (it loaded zeros, but
+            // 0 * inv is a NaN where a tiny range makes inv infinite)
             if ((k & 3) == 0) {
 #pragma unroll
                 for (int i = 0; i < DQF_KS; i++) {
-                    const unsigned q = quantize4(x[i], inv, zpf, nan);
-                    const int v = live && (s0 + i) * 32 + 4 * c8 < k ? (int)q : 0;
+                    const bool in = live && (s0 + i) * 32 + 4 * c8 < k;
+                    bool qnan = false;
+                    const unsigned q = quantize4(x[i], inv, zpf, qnan);
+                    nan |= in && qnan;
+                    const int v = in ? (int)q : 0;
                     sum = __builtin_amdgcn_sdot4(v, 0x01010101, sum, false);
                     dst[i * 256] = v;
                 }

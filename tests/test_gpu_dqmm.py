@@ -412,3 +412,39 @@ def test_dqmm_tile_edges(cuda, oracle, m, k, n, wdt, variant, launches):
         good[m // 2] = False
     assert np.array_equal(acc[good], eacc[good])
     assert np.array_equal(out[good], eo[good])
+
+
+@pytest.mark.parametrize("m,k,n,variant", [
+    (5, 100, 40, 0),                                          # up to 16 rows
+    (20, 100, 40, 0), (33, 36, 129, 0), (40, 516, 130, 0),    # ragged tiles, K % 4 == 0, one and two passes
+    (33, 37, 40, 0), (33, 190, 40, 0),                        # ragged tiles, K % 4 != 0
+    (32, 512, 128, 0), (32, 512, 128, 2),                     # full tiles of 16 and of 32
+    (33, 100, 70, 1), (32, 512, 128, 1),                      # three launches
+])
+def test_dqmm_tiny_range(cuda, oracle, m, k, n, variant):
+    """A range of A so small that 1 / scale is infinite: every value but zero
+    quantizes to 0 or 255, so a row is finite unless it holds a zero (0 * inf).
+    What a tile loads past the matrix (zeros) raises no row's NaN flag."""
+    import ctypes as C
+    from onnxsharp_amd import native as N
+    print(f"dqmm tiny range m={m} k={k} n={n} variant={variant}", flush=True)
+    a = synth.uniform(m + k, (m, k), 3e-38, 3e-37) * np.where(synth.uniform(m * k, (m, k)) < 0.5, -1, 1)
+    a = a.astype(np.float32)
+    a[m - 2, k // 2] = 0.0
+    w = synth.randint(m + n, (k, n), -127, 127, np.int8)
+    ws = synth.uniform(k + n, (n,), 0.001, 0.02)
+    bias = synth.normal(m + k + n, (n,), 0, 0.01)
+    old = C.c_int()
+    N.call("osh_config_get", b"dqmm_variant", C.byref(old))
+    try:
+        N.call("osh_config_set", b"dqmm_variant", variant)
+        out, _, s, z = run_dqmm(cuda, a, w, None, ws, bias)
+    finally:
+        N.call("osh_config_set", b"dqmm_variant", old.value)
+    eo, _, _, es, ez = oracle.dqmm(a, w, None, ws, bias)
+    assert (s, z) == (es, ez) and 0 < s < np.float32(2.9e-39)  # 1 / s overflows
+    good = np.ones(m, bool)
+    good[m - 2] = False
+    assert np.isfinite(eo[good]).all()
+    assert np.array_equal(out[good], eo[good])
+    assert np.isnan(out[m - 2]).all()
