@@ -596,16 +596,22 @@ __device__ __forceinline__ unsigned quantize4(const Quad &x, float inv, float zp
 // (with the checks, the registers of the two load paths are merged by copies
 // that wait for every A load before any B load is issued).
 //
+// KS: k-steps a pass.  All of them are loaded, quantized and staged whatever K
+// is, so a K of at most 4 or 8 steps takes a pass of 4 or 8, with fewer
+// registers and less LDS (16 for every K, then by K): 1352 x 78 x 6499 40.9 ->
+// 21.9 us, 489 x 118 x 212 11.0 -> 8.2, 417 x 96 x 2432 10.8 -> 8.5, 130 x 206 x
+// 3094 11.2 -> 9.7.
+//
 // A and W are not declared __restrict__: the operand loads must stay ahead of
 // the barriers that follow them (the compiler may otherwise sink loads of
 // restrict read-only memory to their first use).
-template <bool FULL>
+template <bool FULL, int KS>
 __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     int m, int k, int n, const float *a, DqScratch *__restrict__ sc, int nparts, int *__restrict__ qparams,
     const int8_t *wpk, const int *__restrict__ colsum, const int *__restrict__ off,
     const float *__restrict__ wscale, int n_wscale, const float *__restrict__ bias, float *__restrict__ out,
     int *__restrict__ acc_out) {
-    __shared__ __attribute__((aligned(16))) int lds_a[DQF_KS * 256];  // [kstep][64 lanes][16 bytes]
+    __shared__ __attribute__((aligned(16))) int lds_a[KS * 256];  // [kstep][64 lanes][16 bytes]
     __shared__ int lds_rs[32], lds_rn[32];
     const int tid = threadIdx.x, lane = tid & 63, wt = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kpad = pad32(k), ks = kpad / 32, npad = pad32(n);
@@ -623,7 +629,7 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     const int row = mt * 32 + r;
     const bool live = FULL || row < m;
     const float *src = a + (long long)(live ? row : 0) * k;
-    const int npass = (ks + DQF_KS - 1) / DQF_KS;
+    const int npass = (ks + KS - 1) / KS;
     const i32x4 *B = reinterpret_cast<const i32x4 *>(wpk) + (long long)(col_live ? nt : 0) * ks * 64 + lane;
 
     // nparts <= 256: one partial per thread (threads past nparts repeat
@@ -635,8 +641,8 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     const bool jlive = col_live && (FULL || j < n);
     const ColOperands col = load_column(j, n, colsum, off, wscale, n_wscale, bias);
 
-    Quad x[DQF_KS];
-    i32x4 b[DQF_KS];
+    Quad x[KS];
+    i32x4 b[KS];
     // Without FULL the loads go through buffer descriptors (of the row tile's
     // rows, of the column tile's k-steps): rows, columns and k-steps that do
     // not exist return zeros and fetch nothing, so every load is unconditional
@@ -651,22 +657,22 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     auto load_pass = [&](int s0) {
         if constexpr (FULL) {
 #pragma unroll
-            for (int i = 0; i < DQF_KS; i++) {
+            for (int i = 0; i < KS; i++) {
                 const float4 v = *reinterpret_cast<const float4 *>(src + (s0 + i) * 32 + 4 * c8);
                 x[i].v[0] = v.x; x[i].v[1] = v.y; x[i].v[2] = v.z; x[i].v[3] = v.w;
             }
 #pragma unroll
-            for (int t = 0; t < DQF_KS; t++) b[t] = B[(s0 + t) * 64];
+            for (int t = 0; t < KS; t++) b[t] = B[(s0 + t) * 64];
         } else {
 #pragma unroll
-            for (int i = 0; i < DQF_KS; i++) {
+            for (int i = 0; i < KS; i++) {
                 const int kk = (s0 + i) * 32 + 4 * c8;
                 const auto v = __builtin_amdgcn_raw_buffer_load_b128(ra, kk < k ? (r * k + kk) * 4 : -1, 0, 0);
 #pragma unroll
                 for (int e = 0; e < 4; e++) x[i].v[e] = __uint_as_float(v[e]);
             }
 #pragma unroll
-            for (int t = 0; t < DQF_KS; t++) {
+            for (int t = 0; t < KS; t++) {
                 const auto v = __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + (s0 + t) * 1024, 0, 0);
                 b[t] = i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
             }
@@ -690,17 +696,17 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
     i32x16 acc0 = {}, acc1 = {};
     int *dst = lds_a + (r + 32 * (c8 >> 2)) * 4 + (c8 & 3);
     for (int ps = 0; ps < npass; ps++) {
-        const int s0 = ps * DQF_KS;
+        const int s0 = ps * KS;
         if constexpr (FULL) {
 #pragma unroll
-            for (int i = 0; i < DQF_KS; i++) dst[i * 256] = (int)quantize4(x[i], inv, zpf, 0xfu, sum, nan);
+            for (int i = 0; i < KS; i++) dst[i * 256] = (int)quantize4(x[i], inv, zpf, 0xfu, sum, nan);
         } else {
             // k % 4 == 0: a quad is all inside its row or not there at all, so
             // one select masks it, and one its NaN flag (it loaded zeros, but
             // 0 * inv is a NaN where a tiny range makes inv infinite)
             if ((k & 3) == 0) {
 #pragma unroll
-                for (int i = 0; i < DQF_KS; i++) {
+                for (int i = 0; i < KS; i++) {
                     const bool in = live && (s0 + i) * 32 + 4 * c8 < k;
                     bool qnan = false;
                     const unsigned q = quantize4(x[i], inv, zpf, qnan);
@@ -711,7 +717,7 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
                 }
             } else {
 #pragma unroll
-                for (int i = 0; i < DQF_KS; i++) {
+                for (int i = 0; i < KS; i++) {
                     const int kk = (s0 + i) * 32 + 4 * c8;
                     unsigned lm = 0;
 #pragma unroll
@@ -723,18 +729,18 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
         __syncthreads();
         {
             const int *srcl = lds_a + lane * 4;
-            if (FULL || s0 + DQF_KS <= ks) {  // k-steps past the last are zeros
-                i32x4 av[DQF_KS];
+            if (FULL || s0 + KS <= ks) {  // k-steps past the last are zeros
+                i32x4 av[KS];
 #pragma unroll
-                for (int t = 0; t < DQF_KS; t++) av[t] = *reinterpret_cast<const i32x4 *>(srcl + t * 256);
+                for (int t = 0; t < KS; t++) av[t] = *reinterpret_cast<const i32x4 *>(srcl + t * 256);
 #pragma unroll
-                for (int t = 0; t < DQF_KS; t += 2) {
+                for (int t = 0; t < KS; t += 2) {
                     acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[t], b[t], acc0, 0, 0, 0);
                     acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[t + 1], b[t + 1], acc1, 0, 0, 0);
                 }
             } else {
 #pragma unroll
-                for (int t = 0; t < DQF_KS; t++) {
+                for (int t = 0; t < KS; t++) {
                     if (s0 + t < ks) {
                         const i32x4 av = *reinterpret_cast<const i32x4 *>(srcl + t * 256);
                         if (t & 1) acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, b[t], acc1, 0, 0, 0);
@@ -747,7 +753,7 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
             // the next pass's loads go out after this pass's MFMAs, whose b
             // registers they reuse
             __builtin_amdgcn_sched_barrier(0);
-            load_pass(s0 + DQF_KS);  // x and b are free: the pass is quantized and multiplied
+            load_pass(s0 + KS);  // x and b are free: the pass is quantized and multiplied
             __syncthreads();         // every wave's MFMAs have read the pass before it is rewritten
         }
     }
@@ -1203,13 +1209,18 @@ static osh_status dqmm_run(int m, int k, int n, const float *d_a, const void *d_
                        d_a, sc, nparts, (int *)d_qparams, frag, colsum, off, d_wscale, n_wscale, d_bias, d_out,
                        (int *)d_acc);
         else if (full)
-            OSH_LAUNCH(dqmm_fused_kernel<true>, dim3((unsigned)fblocks), dim3(64 * DQF_WAVES), 0, st, m, k, n,
+            OSH_LAUNCH((dqmm_fused_kernel<true, DQF_KS>), dim3((unsigned)fblocks), dim3(64 * DQF_WAVES), 0, st, m, k, n,
                                d_a, sc, nparts, (int *)d_qparams, frag, colsum, off, d_wscale, n_wscale, d_bias, d_out,
                                (int *)d_acc);
-        else
-            OSH_LAUNCH(dqmm_fused_kernel<false>, dim3((unsigned)fblocks), dim3(64 * DQF_WAVES), 0, st, m, k,
-                               n, d_a, sc, nparts, (int *)d_qparams, frag, colsum, off, d_wscale, n_wscale, d_bias,
-                               d_out, (int *)d_acc);
+        else {
+#define OSH_RAGGED(KS)                                                                                               \
+    OSH_LAUNCH((dqmm_fused_kernel<false, KS>), dim3((unsigned)fblocks), dim3(64 * DQF_WAVES), 0, st, m, k, n, d_a, sc, \
+               nparts, (int *)d_qparams, frag, colsum, off, d_wscale, n_wscale, d_bias, d_out, (int *)d_acc)
+            if (k <= 4 * 32) OSH_RAGGED(4);
+            else if (k <= 8 * 32) OSH_RAGGED(8);
+            else OSH_RAGGED(DQF_KS);
+#undef OSH_RAGGED
+        }
         OSH_LAUNCH_CHECK("dqmm_fused_kernel");
         t_dqmm_launches = 2;
         return OSH_OK;

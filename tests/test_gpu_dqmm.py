@@ -372,6 +372,9 @@ def _no_acc_case(cuda, oracle, m, k, n, noalloc, offset):
     (16, 2050, 96, np.uint8, 0, 2),
     # ragged tiles of the fused launch: one past a tile, k % 4 != 0, two and three passes
     (17, 36, 129, np.int8, 0, 2), (33, 513, 127, np.uint8, 0, 2), (65, 1100, 130, np.int8, 0, 2),
+    # and at most 4, at most 8 and 9 or more k-steps
+    (17, 127, 40, np.uint8, 0, 2), (33, 128, 33, np.int8, 0, 2), (40, 129, 130, np.int8, 0, 2),
+    (20, 255, 70, np.int8, 0, 2), (64, 256, 129, np.uint8, 0, 2), (35, 257, 64, np.uint8, 0, 2),
     # three launches, 32-row tiles: one and several stages, ragged in each direction
     (31, 33, 127, np.uint8, 1, 3), (33, 128, 129, np.int8, 1, 3), (65, 1157, 257, np.uint8, 1, 3),
     # 64-row tiles (enough workgroups), and the size rule's own choice of three launches
