@@ -92,8 +92,10 @@ struct G16B {
 };
 
 // Epilogue of a (16 * TM) x (16 * BV * TN) wave tile: column scale (fmaf),
-// activation, residual, BV-wide accesses (any 4-byte address will do).  RAG
-// (N % BV != 0) stores the columns of a vector that crosses N one by one; it is
+// activation, residual, BV-wide accesses (any 4-byte address will do).  A lane's
+// four rows get their values before the first is stored: a use of the column
+// operands between the stores waits for the store before it (13 x 96 x 4256
+// 3.51 us, so 3.23).  RAG (N % BV != 0) stores the columns of a vector that crosses N one by one; it is
 // a template parameter because that code beside the other, reached or not, cost
 // the compiler's schedule of the main loop (4096 x 1024 x 4096 247 -> 321 us).
 template <int TM, int TN, int BV, int ACT, bool RAG>
@@ -113,17 +115,20 @@ __device__ __forceinline__ void g16_store(const IgemmArgs &p, const f32x4 (&acc)
                 cs[q] = p.col_scale ? p.col_scale[cq] : 0.f;
                 cb[q] = (p.col_scale && p.col_bias) ? p.col_bias[cq] : 0.f;
             }
+            float v[4][BV];
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int q = 0; q < BV; q++) {
+                    v[r][q] = acc[tm][tn * BV + q][r];
+                    if (p.col_scale) v[r][q] = __builtin_fmaf(v[r][q], cs[q], cb[q]);
+                    v[r][q] = activate<ACT>(v[r][q]);
+                }
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int row = m0 + 16 * tm + 4 * g + r;
                 if (row >= M) continue;
-                float o[BV];
-#pragma unroll
-                for (int q = 0; q < BV; q++) {
-                    float v = acc[tm][tn * BV + q][r];
-                    if (p.col_scale) v = __builtin_fmaf(v, cs[q], cb[q]);
-                    o[q] = activate<ACT>(v);
-                }
+                float(&o)[BV] = v[r];
                 const long long at = (long long)row * p.ldc + col;
                 if (!RAG || col + BV <= N) {
                     if (R) {
