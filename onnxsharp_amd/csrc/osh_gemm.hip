@@ -40,12 +40,12 @@ int osh::gemm16_variant_count() { return kG16Count; }
 
 namespace osh {
 
-// Every wave tile takes any alignment, stride and remainder (osh_gemm16.h):
-// what is left is K >= 1 and 32-bit buffer offsets, also those of the k past K
-// that a tail chunk asks for.  Before, odd rows (lda or ldb not a multiple of
-// the load width) went to igemm_f32_kernel, whose guarded loads wait for each
-// other: 484 x 2468 x 7063 322 -> 159 us, 8 x 3653 x 74 168 -> 21 us, 1929 x
-// 3986 x 41 217 -> 51 us.
+// Every wave tile takes any alignment, stride and remainder of rows at least BV
+// columns wide (osh_gemm16.h): what is left is K >= 1 and 32-bit buffer offsets,
+// also those of the k past K that a tail chunk asks for.  Before, odd rows (lda
+// or ldb not a multiple of the load width) went to igemm_f32_kernel, whose
+// guarded loads wait for each other: 484 x 2468 x 7063 322 -> 159 us, 8 x 3653 x
+// 74 168 -> 21 us, 1929 x 3986 x 41 217 -> 51 us.
 static bool g16_fits(const IgemmArgs &a) {
     const long long kmax = a.K + 64LL;
     return a.K >= 1 && ((a.M - 1LL) * a.lda + kmax) * 4 < (1LL << 31) && (kmax * a.ldb + a.N + 64) * 4 < (1LL << 31);
@@ -83,13 +83,8 @@ static osh_status g16_launch(const IgemmArgs &a, int zcount, int act, hipStream_
     const long long blocks = (long long)ceil_div(tiles_m, 4) * tiles_n;
     if (blocks > 0x7fffffffLL) return fail(OSH_E_UNSUPPORTED, "GEMM grid too large");
     dim3 grid((unsigned)blocks, zcount);
-    if (a.N % BV) {
-        OSH_DISPATCH_ACT(act, ACT, OSH_LAUNCH((gemm16_kernel<TM, TN, BV, KC, ACT, (BV > 1)>), grid, dim3(256), 0, st,
-                                              a, tiles_m));
-    } else {
-        OSH_DISPATCH_ACT(act, ACT,
-                         OSH_LAUNCH((gemm16_kernel<TM, TN, BV, KC, ACT, false>), grid, dim3(256), 0, st, a, tiles_m));
-    }
+    OSH_DISPATCH_ACT(act, ACT,
+                     OSH_LAUNCH((gemm16_kernel<TM, TN, BV, KC, ACT>), grid, dim3(256), 0, st, a, tiles_m));
     OSH_LAUNCH_CHECK("gemm16_kernel");
     return OSH_OK;
 }
@@ -97,14 +92,15 @@ static osh_status g16_launch(const IgemmArgs &a, int zcount, int act, hipStream_
 // Returns true when a gemm16 tile took the problem (*status = its launch status).
 static bool launch_gemm16(const IgemmArgs &a, int zcount, int act, hipStream_t st, osh_status *status) {
     const int forced = gemm_variant();
-    if (forced == -2 || zcount > 65535 || !g16_fits(a)) return false;
+    if (forced == -2 || forced >= kG16Count || zcount > 65535 || !g16_fits(a)) return false;
     int best = -1;
-    if (forced >= 0) {
-        if (forced < kG16Count) best = forced;
+    if (forced >= 0 && a.N >= kG16[forced].bv) {
+        best = forced;
     } else {
         const int cus = device_cus();
         double bc = 0;
         for (int i = 0; i < kG16Count; i++) {
+            if (a.N < kG16[i].bv) continue;
             const double c = g16_cost(a, zcount, kG16[i], cus);
             if (best < 0 || c < bc) best = i, bc = c;
         }

@@ -29,12 +29,13 @@
 //     of B[k0 + 4s + g][col .. col + BV - 1], col = 16*BV*tn + BV*j; component
 //     q feeds output block q of the tile, whose column j stands for col + q, so
 //     a lane stores BV adjacent columns at once.
-// k offsets live in scalar registers, or in the vector offset where a load may
-// reach past its operand (osh_gemm16_addr.h).  Loads go through buffer
-// descriptors, so 4-byte alignment is enough for every width and no load sits
-// under a condition: rows past M are clamped, columns past N computed and never
-// stored, the K tail (K % KC) zero-filled, and a zero product leaves the chain
-// unchanged.
+// k offsets live in scalar registers, in the chunk that K ends in in the vector
+// offset (osh_gemm16_addr.h).  Loads go through buffer descriptors, so 4-byte
+// alignment is enough for every width and no load sits under a condition: rows
+// past M are clamped; a lane whose BV columns would cross N takes the last BV
+// columns, some of which its neighbour computes and stores too, to the same bits;
+// one whose columns start past N stores nothing; the K tail (K % KC) is
+// zero-filled, and a zero product leaves the chain unchanged.
 #pragma once
 
 #include <type_traits>
@@ -95,10 +96,8 @@ struct G16B {
 // activation, residual, BV-wide accesses (any 4-byte address will do).  A lane's
 // four rows get their values before the first is stored: a use of the column
 // operands between the stores waits for the store before it (13 x 96 x 4256
-// 3.51 us, so 3.23).  RAG (N % BV != 0) stores the columns of a vector that crosses N one by one; it is
-// a template parameter because that code beside the other, reached or not, cost
-// the compiler's schedule of the main loop (4096 x 1024 x 4096 247 -> 321 us).
-template <int TM, int TN, int BV, int ACT, bool RAG>
+// 3.51 us, so 3.23).
+template <int TM, int TN, int BV, int ACT>
 __device__ __forceinline__ void g16_store(const IgemmArgs &p, const f32x4 (&acc)[TM][TN * BV], int m0, int n0, int j,
                                           int g, float *__restrict__ C, const float *__restrict__ R) {
     const int M = p.M, N = p.N;
@@ -106,14 +105,13 @@ __device__ __forceinline__ void g16_store(const IgemmArgs &p, const f32x4 (&acc)
     for (int tm = 0; tm < TM; tm++)
 #pragma unroll
         for (int tn = 0; tn < TN; tn++) {
-            const int col = n0 + 16 * BV * tn + BV * j;
-            if (col >= N) continue;
+            if (n0 + 16 * BV * tn + BV * j >= N) continue;
+            const int col = g16_col<BV>(n0 + 16 * BV * tn + BV * j, N);
             float cs[BV], cb[BV];
 #pragma unroll
             for (int q = 0; q < BV; q++) {
-                const int cq = RAG ? min(col + q, N - 1) : col + q;
-                cs[q] = p.col_scale ? p.col_scale[cq] : 0.f;
-                cb[q] = (p.col_scale && p.col_bias) ? p.col_bias[cq] : 0.f;
+                cs[q] = p.col_scale ? p.col_scale[col + q] : 0.f;
+                cb[q] = (p.col_scale && p.col_bias) ? p.col_bias[col + q] : 0.f;
             }
             float v[4][BV];
 #pragma unroll
@@ -130,24 +128,18 @@ __device__ __forceinline__ void g16_store(const IgemmArgs &p, const f32x4 (&acc)
                 if (row >= M) continue;
                 float(&o)[BV] = v[r];
                 const long long at = (long long)row * p.ldc + col;
-                if (!RAG || col + BV <= N) {
-                    if (R) {
-                        float t[BV];
-                        __builtin_memcpy(t, R + at, sizeof(t));
+                if (R) {
+                    float t[BV];
+                    __builtin_memcpy(t, R + at, sizeof(t));
 #pragma unroll
-                        for (int q = 0; q < BV; q++) o[q] += t[q];
-                    }
-                    __builtin_memcpy(C + at, o, sizeof(o));
-                } else {
-#pragma unroll
-                    for (int q = 0; q < BV; q++)
-                        if (col + q < N) C[at + q] = R ? o[q] + R[at + q] : o[q];
+                    for (int q = 0; q < BV; q++) o[q] += t[q];
                 }
+                __builtin_memcpy(C + at, o, sizeof(o));
             }
         }
 }
 
-template <int TM, int TN, int BV, int KC, int ACT, bool RAG>
+template <int TM, int TN, int BV, int KC, int ACT>
 __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
     constexpr int STEPS = KC / 4;
     constexpr int AU = KC / 16;  // A float4 slots per lane per 16-row block
@@ -190,14 +182,14 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
     const int lr = j * 16 + g * 4;  // lane (j, g) reads [tm][kg][j][g][0..3]
     int vob[TN];
 #pragma unroll
-    for (int tn = 0; tn < TN; tn++) vob[tn] = g16_lane_b(g, n0 + 16 * BV * tn + BV * j, N, ldb);
+    for (int tn = 0; tn < TN; tn++) vob[tn] = g16_lane_b(g, g16_col<BV>(n0 + 16 * BV * tn + BV * j, N), ldb);
 
     f32x4 acc[TM][TN * BV];
 #pragma unroll
     for (int tn = 0; tn < TN; tn++)
 #pragma unroll
         for (int q = 0; q < BV; q++) {
-            const int col = min(n0 + 16 * BV * tn + BV * j + q, N - 1);
+            const int col = g16_col<BV>(n0 + 16 * BV * tn + BV * j, N) + q;
             const float cb = (!p.col_scale && p.col_bias) ? p.col_bias[col] : 0.f;
 #pragma unroll
             for (int tm = 0; tm < TM; tm++)
@@ -232,7 +224,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
         for (int s = 0; s < STEPS; s++)
 #pragma unroll
             for (int tn = 0; tn < TN; tn++) {
-                const G16Off o = g16_off_b<decltype(tail)::value, RAG>(vob[tn], c * KC + 4 * s, ldb);
+                const G16Off o = g16_off_b<decltype(tail)::value>(vob[tn], c * KC + 4 * s, ldb);
                 R.v[s][tn] = g16_load_b<BV>(rb, o.vec, o.scalar);
             }
     };
@@ -351,7 +343,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(IgemmArgs p, int tiles_m) {
         compute(av, rb);
     }
 
-    g16_store<TM, TN, BV, ACT, RAG>(p, acc, m0, n0, j, g, C, R);
+    g16_store<TM, TN, BV, ACT>(p, acc, m0, n0, j, g, C, R);
 }
 
 }  // namespace osh

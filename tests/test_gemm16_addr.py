@@ -2,10 +2,11 @@
 arithmetic (csrc/osh_gemm16_addr.h, plain C++ on the host) is enumerated over
 every tile, lane and chunk at the remainders of M, K and N.
 
-A word of a buffer load is fetched when its vector offset lies below the
-descriptor's size, at vector + scalar offset.  Every word fetched must lie in
-the operand, and every word the product needs must be fetched, from where the
-matrix holds it."""
+A word of a buffer load is fetched, at vector + scalar offset, when the offset
+lies below the descriptor's size: the vector offset alone or (as gfx950 does it)
+vector plus scalar.  Every word that the looser reading fetches must lie in the
+operand, and every word the product needs must be fetched under the stricter one,
+from where the matrix holds it."""
 import os
 import re
 import shutil
@@ -29,8 +30,8 @@ static void check(G16Off o, int words, int bytes, const bool *need, const int *a
     loads++;
     for (int q = 0; q < words; q++) {
         const long long v = (unsigned)o.vec + 4LL * q, a = (long long)o.vec + o.scalar + 4 * q;
-        const bool fetched = v < bytes;
-        if ((fetched && (a < 0 || a + 4 > bytes)) || (need[q] && (!fetched || a != at[q]))) {
+        const bool may = v < bytes, does = v + (unsigned)o.scalar < bytes;
+        if ((may && (a < 0 || a + 4 > bytes)) || (need[q] && (!does || a != at[q]))) {
             printf("%s of tile %d, %d x %d x %d, lda %d, ldb %d: word at byte %lld of %d %s\n", what, tile, M, K, N, lda,
                    ldb, a, bytes, need[q] ? "is not the one needed" : "lies outside");
             exit(1);
@@ -55,19 +56,35 @@ static void chunk_a(int c, int rows, int kc) {  // the kernel clamps rows to M -
         }
 }
 
-template <bool TAIL, bool RAG>
+static int first_column(int bv, int col) {
+    return bv == 1 ? g16_col<1>(col, N) : bv == 2 ? g16_col<2>(col, N) : bv == 3 ? g16_col<3>(col, N) : g16_col<4>(col, N);
+}
+
+template <bool TAIL>
 static void chunk_b(int c, int cols, int bv, int kc) {
     what = "B";
     const int bytes = g16_bytes_b(K, N, ldb);
     for (int s = 0; s < kc / 4; s++)
         for (int g = 0; g < 4; g++)
             for (int col = 0; col < cols; col += bv) {
-                const int k = c * kc + 4 * s + g;
+                const int k = c * kc + 4 * s + g, first = first_column(bv, col);
                 bool need[4];
                 int at[4];
-                for (int q = 0; q < bv; q++) need[q] = k < K && col + q < N, at[q] = (k * ldb + col + q) * 4;
-                check(g16_off_b<TAIL, RAG>(g16_lane_b(g, col, N, ldb), c * kc + 4 * s, ldb), bv, bytes, need, at);
+                for (int q = 0; q < bv; q++) need[q] = k < K && col < N, at[q] = (k * ldb + first + q) * 4;
+                check(g16_off_b<TAIL>(g16_lane_b(g, first, ldb), c * kc + 4 * s, ldb), bv, bytes, need, at);
             }
+}
+
+// Every column is stored, by lanes whose columns all exist.
+static void columns(int cols, int bv) {
+    bool stored[512] = {};
+    for (int col = 0; col < cols && col < N; col += bv)
+        for (int q = 0; q < bv; q++) stored[first_column(bv, col) + q] = true;
+    for (int j = 0; j < 512; j++)
+        if (stored[j] != (j < N)) {
+            printf("tile %d, N %d: column %d %s\n", tile, N, j, stored[j] ? "does not exist" : "is not stored");
+            exit(1);
+        }
 }
 
 int main() {
@@ -82,11 +99,11 @@ int main() {
                         M = m, N = n, lda = K + pad, ldb = N + 2 * pad;
                         const int rows = (M + 16 * tm - 1) / (16 * tm) * 16 * tm;
                         const int cols = (N + 16 * bv * tn - 1) / (16 * bv * tn) * 16 * bv * tn;
+                        if (M == ms[0] && N >= bv) columns(cols, bv);
                         for (int c = 0; c * kc < K; c++) {
-                            const bool tail = (c + 1) * kc > K, rag = N % bv != 0;
+                            const bool tail = (c + 1) * kc > K;
                             if (N == ns[0]) tail ? chunk_a<true>(c, rows, kc) : chunk_a<false>(c, rows, kc);
-                            if (M == ms[0] && tail) rag ? chunk_b<true, true>(c, cols, bv, kc) : chunk_b<true, false>(c, cols, bv, kc);
-                            if (M == ms[0] && !tail) rag ? chunk_b<false, true>(c, cols, bv, kc) : chunk_b<false, false>(c, cols, bv, kc);
+                            if (M == ms[0] && N >= bv) tail ? chunk_b<true>(c, cols, bv, kc) : chunk_b<false>(c, cols, bv, kc);
                         }
                     }
         tile++;
