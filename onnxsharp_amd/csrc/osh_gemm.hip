@@ -51,30 +51,35 @@ static bool g16_fits(const IgemmArgs &a) {
     return a.K >= 1 && ((a.M - 1LL) * a.lda + kmax) * 4 < (1LL << 31) && (kmax * a.ldb + a.N + 64) * 4 < (1LL << 31);
 }
 
-// Predicted time of a wave tile, in cycles up to a common factor.  A wave's
-// chunk takes its MFMAs or, where those are fewer, one trip to memory (loads are
-// one chunk ahead): 600 in L2, 715 past it, for 32 k; 64-k chunks pay only where
-// the operands (A and B together) are well past the 4 MB of an XCD's L2, since
-// their 16 MFMAs a block are no shorter a chain (6 MB: at 4.3 MB 64-k chunks cost
-// 62 x 1984 x 480 14.3 -> 16.7 us with both operands in L2, and gave 13 x 417 x
-// 2572 8.0 -> 7.0 without).  Waves beyond one a SIMD
-// add their MFMAs, and part of their prologue and epilogue, which overlap.
+// Predicted time of a wave tile, in cycles, less what all tiles share.  A wave's
+// chunk takes its MFMAs (32 cycles each, 90 more a chunk) or, where those are
+// fewer, one trip past L2 (loads are one chunk ahead).  64-k chunks pay only for
+// such trips, of small waves: their MFMAs are no fewer, their prologue is longer.
+// Whether the operands (A and B together) come from past L2 is put at 6 MB.  What
+// a program that multiplies by other weights in between sees is the cold side: 7 x
+// 480 x 3840 8.6 us with 16 x 16 tiles of 32 k, 7.1 of 64 k, 14 x 3584 x 480 41.7
+// and 25.9; the same operands again and again, in L2, take 5.7 and 6.5, 20.6 and 25.
+// Further waves of a SIMD add their MFMAs (its pipe is full by then, so a little
+// less than 32 cycles each), address and LDS work, prologue and epilogue (more
+// for two row blocks); their number is half way between the average and the
+// fullest SIMD's, since workgroups that end early make room for others.
 // Workgroups of four waves fill the chip by fours, so slots count, not tiles
 // (of fewer row tiles the idle waves leave at once).
-// Fitted to 180 products (m 1-4096, k 32-4096, n 32-8192): on average 1.8% above
-// the best tile of each, the former rule (rounds of waves times MFMAs, inflated
-// by loads an MFMA) 6.8% and up to 57% (208 x 2952 x 1226 66 -> 42 us, 16 x 3566
-// x 1223 43 -> 28, 820 x 384 x 1760 25 -> 17).
+// Fitted to 979 products and batches (m 1-4096, k 32-4096, n 32-8192), each with
+// its operands in L2 and out of it: on average 0.9% and 2.1% above the best tile
+// (an earlier fit with hardly a term for the fullest SIMD 1.6% and 2.8%, its 64-k
+// tiles among several waves a SIMD up to 36% slower: 1946 x 448 x 2560 58.1 ->
+// 45.5 us, 14 of 436 x 128 x 436 19.2 -> 14.2).
 static double g16_cost(const IgemmArgs &a, int zcount, const G16Variant &v, int cus) {
     const int tiles_m = ceil_div(a.M, 16 * v.tm), waves = std::min(tiles_m, 4);
     const double slots = (double)ceil_div(tiles_m, waves) * waves * ceil_div(a.N, 16 * v.bv * v.tn) * zcount;
-    const double u = (double)v.tm * v.tn * v.bv;
+    const double u = (double)v.tm * v.tn * v.bv, k32 = v.kc / 32.0;
     const bool far = 4.0 * zcount * ((double)a.M * a.K + (double)a.K * a.N) > 6e6;
-    const double chunks = ceil_div(a.K, v.kc), mfma = v.kc / 4 * 22.0 * u;
-    const double trip = v.kc == 32 ? (far ? 715 : 600) : (far ? 1270 + 60 * u : 4000);
+    const double chunks = ceil_div(a.K, v.kc), trip = v.kc == 32 ? (far ? 700 : 0) : (far ? 850 : 3000);
     const double per_simd = slots / (4.0 * cus);
-    const double more = std::max(0.0, 0.2 * std::ceil(per_simd) + 0.8 * per_simd - 1.0);
-    return 3800 + 450 * u + chunks * std::max(trip, mfma + 60) + more * (1.15 * chunks * mfma + 270 * u);
+    const double more = std::max(0.0, 0.5 * std::ceil(per_simd) + 0.5 * per_simd - 1.0);
+    return 1500 * u + (v.kc == 64 ? 3500 : 0) + chunks * std::max(trip, 90 + 256 * u * k32) +
+           more * (chunks * k32 * (230 * u + 450) + 1000 * u + 300 + 4500 * (v.tm - 1));
 }
 
 template <int TM, int TN, int BV, int KC>

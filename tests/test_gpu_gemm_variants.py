@@ -153,3 +153,22 @@ def test_gemm_variant_option_range():
     from onnxsharp_amd import native as N
     with pytest.raises(N.OshError):
         N.call("osh_config_set", b"gemm_variant", 1000)
+
+
+@pytest.mark.parametrize("batch,m,k,n,kc", [
+    (1, 1946, 448, 2560, 32), (1, 207, 448, 5376, 32), (14, 436, 128, 436, 32), (1, 1881, 300, 7796, 32),  # 3 to 20 waves a SIMD
+    (1, 16, 3566, 1223, 64), (1, 4, 3040, 4960, 64),  # a few waves, each waiting for memory
+])
+def test_gemm_chunk_length_rule(cuda, batch, m, k, n, kc):
+    """64-k chunks hide a wave's own trips to memory and are for products of few
+    waves: where a SIMD has several, the tile is one of 32-k chunks."""
+    import torch
+    from onnxsharp_amd import native as N
+    a, b, c = (torch.zeros(s, device=cuda) for s in ((batch, m, k), (batch, k, n), (batch, m, n)))
+    ptr = lambda t: C.c_void_p(t.data_ptr())
+    N.kernel_log(reset=True)
+    N.call("osh_gemm_f32_batched", batch, m, n, k, ptr(a), k, m * k, ptr(b), n, k * n, None, 0, ptr(c), n, m * n,
+           C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    names = N.kernel_log(reset=True)
+    assert len(names) == 1 and names[0].startswith("gemm16_kernel<") and int(names[0].split(",")[3]) == kc, names
