@@ -30,11 +30,11 @@
 //
 // Bound by what the L2s deliver: 8 x 64 x 56 x 56 -> 64 with a residual reads
 // 215 MB through L1 with one output block a workgroup (weights once per 16
-// tiles, patches once per 16 channels), 160 with two, at about 15 TB/s: 24.1
-// and 22.9 us (31.9 before, its patch loads and stores one guarded value at a
-// time).  Workgroups of 32 tiles (weights shared through L1) 26.5 and 24.0; all
-// 16 components x 32 x 32 in four waves 33.6 (registers); patches two chunks
-// ahead no change.
+// tiles, patches once per 16 channels), 160 with two, at about 15 TB/s: 21.3 us
+// with either (33.5 with patch loads and stores one guarded value at a time; 24.1
+// and 22.5 when the last chunks were not yet apart, which showed workgroups of 32
+// tiles, weights shared through L1, slower by 5-10%, all 16 components x 32 x 32
+// in four waves by 40% (registers), patches two chunks ahead no change).
 #pragma once
 
 #include "osh_common.h"
@@ -223,7 +223,8 @@ __global__ __launch_bounds__(256 * OB, 4) void wino_f23_kernel(osh_conv_params p
     }
     load_u(w1, 1);
     __syncthreads();
-    for (int ch = 0; ch < cbs; ch += 2) {
+    int ch = 0;
+    for (; ch + 2 < cbs; ch += 2) {
         // planes of chunk ch in buffer 0; pa and w1 hold chunk ch + 1
         multiply(w0, lds[0]);
         load_u(w0, ch + 2);
@@ -232,7 +233,6 @@ __global__ __launch_bounds__(256 * OB, 4) void wino_f23_kernel(osh_conv_params p
             load_patch(pa, ch + 2);
         }
         __syncthreads();
-        if (ch + 1 >= cbs) break;
         multiply(w1, lds[1]);
         load_u(w1, ch + 3);
         if (transforms) {
@@ -241,6 +241,16 @@ __global__ __launch_bounds__(256 * OB, 4) void wino_f23_kernel(osh_conv_params p
         }
         __syncthreads();
     }
+    // the last one or two chunks, with nothing left to load or, after them, to
+    // transform (a chunk too many, of zeros, cost 4 x 8 x 33 x 28 -> 168 6.9 us;
+    // 6.0 so)
+    multiply(w0, lds[0]);
+    if (ch + 1 < cbs) {
+        if (transforms) transform_store(pa, lds[1]);
+        __syncthreads();
+        multiply(w1, lds[1]);
+    }
+    __syncthreads();
     // accumulators -> [comp][oc][tile]; D[row 4g + r][col j]
     float *ms = lds[0];
     {
