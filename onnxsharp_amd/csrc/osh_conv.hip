@@ -1085,9 +1085,9 @@ static osh_status conv2d(const osh_conv_params *p, const float *d_x, const void 
             // Two output blocks a workgroup where that still gives most CUs
             // one: 8 x 256 x 14 x 14 -> 256 (200 workgroups) 18.4 us (one block
             // 20.8), 2 x 64 x 13 x 74 -> 200 (231) 7.2 (8.0); 2 x 128 x 28 x 28 ->
-            // 128 (100) 10.2 (8.4).  Past one workgroup a CU the two are within 10%
-            // of each other either way: 2 x 40 x 70 x 24 -> 240 (424) 9.3 (10.8), 4 x
-            // 8 x 33 x 28 -> 168 (360) 5.9 (5.6).
+            // 128 (100) 10.2 (8.4).  Past one workgroup a CU either can win: 2 x
+            // 40 x 70 x 24 -> 240 (424) 9.3 (10.8), 8 x 64 x 56 x 56 -> 64 (784) 21.4
+            // (21.3), 4 x 64 x 14 x 43 -> 200 (273) 10.4 (8.6).
             if (p->m > 16 && (tiles + 15) / 16 * ((p->m + 31) / 32) >= 5 * device_cus() / 8) OSH_WINO(2);
             else OSH_WINO(1);
             OSH_LAUNCH_CHECK("wino_f23_kernel");

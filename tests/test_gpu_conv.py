@@ -218,7 +218,7 @@ RESIDUAL_CASES = [
     ("pw_gemm_tile_1x1_64to48_40", (1, 64, 40, 40), (48, 64, 1, 1), dict(), 0),
     ("pw_lds_tile_1x1_80to64_20x24", (2, 80, 20, 24), (64, 80, 1, 1), dict(), 5),
     ("pw_lds_tile_1x1_48to32_odd", (1, 48, 17, 19), (32, 48, 1, 1), dict(), 3),
-    ("igemm_1x1_c6_odd", (2, 6, 13, 11), (10, 6, 1, 1), dict(), -1),
+    ("gemm_tile_1x1_c6_odd", (2, 6, 13, 11), (10, 6, 1, 1), dict(), -1),
     ("direct3x3_c8_160", (1, 8, 160, 160), (16, 8, 3, 3), dict(pads=[1, 1, 1, 1]), -1),
     ("depthwise_64_20", (1, 64, 20, 20), (64, 1, 3, 3), dict(group=64, pads=[1, 1, 1, 1]), -1),
     ("first_conv_c3", (1, 3, 64, 64), (16, 3, 3, 3), dict(pads=[1, 1, 1, 1]), -1),

@@ -103,6 +103,51 @@ def test_gemm_variants_ragged_rows(cuda, oracle, variant_reset, m, k, n, off):
         assert np.array_equal(y[off:].reshape(m, ldc)[:, :n], ref), f"variant {v}: not bit-identical"
 
 
+@pytest.mark.parametrize("m,k,n", [(17, 33, 5), (35, 19, 50), (16, 65, 67), (33, 70, 131)])
+def test_gemm_variants_ragged_epilogues(cuda, oracle, variant_reset, m, k, n):
+    """Rows that end inside a lane's columns through every epilogue of every
+    tile: column scale and bias, a residual (a 1x1 conv's; the lanes of a row's
+    end write some columns twice), and batches at odd strides."""
+    import torch
+    from onnxsharp_amd import native as N
+    from onnxsharp_amd.layers import ConvLayer
+    batch = 3
+    a = synth.uniform(m * 13 + k, (batch, m, k), -1, 1)
+    b = synth.uniform(n * 17 + k, (batch, k, n), -1, 1)
+    cs, cb = synth.uniform(m + n, (n,), 1e-3, 1e-1), synth.uniform(m + k, (n,), -1, 1)
+    rb, res = synth.uniform(n + k, (m,), -1, 1), synth.uniform(m + n + k, (batch, m, n), -1, 1)
+    st = lambda: C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ptr = lambda t: C.c_void_p(t.data_ptr())
+    ref_scale = oracle.relu(oracle.gemm_f32(a[0], b[0], col_bias=cb, col_scale=cs))
+    ref_batch = np.stack([oracle.gemm_f32(a[i], b[i], col_bias=cb) for i in range(batch)])
+    ref_conv = np.stack([oracle.gemm_f32(a[0], b[i], row_bias=rb) + res[i] for i in range(batch)])
+
+    def strided(x, stride):
+        buf = np.full((x.shape[0], stride), np.nan, np.float32)
+        buf[:, :x[0].size] = x.reshape(x.shape[0], -1)
+        return _t(buf, cuda)
+
+    sa, sb, sc = m * k + 1, k * n + 3, m * n + 1
+    da, db, dcb = strided(a, sa), strided(b, sb), _t(cb, cuda)
+    layer = ConvLayer(group=1, strides=[1, 1], pads=[0] * 4)
+    dx, dw, drb, dres = (_t(v, cuda) for v in (b.reshape(batch, k, 1, n), a[0].reshape(m, k, 1, 1), rb,
+                                               res.reshape(batch, m, 1, n)))
+    for v in _variants() + [-1]:
+        print(f"gemm variant {v}: ragged epilogues m={m} k={k} n={n}", flush=True)
+        N.call("osh_config_set", b"gemm_variant", v)
+        y = _gemm(cuda, m, k, n, k, n + 1, a[0], b[0], col_bias=cb, col_scale=cs, act=N.ACT_RELU)
+        assert np.array_equal(y, ref_scale), f"variant {v}: column scale"
+        dc = torch.full((batch, sc), 7.0, device=cuda)
+        N.call("osh_gemm_f32_batched", batch, m, n, k, ptr(da), k, sa, ptr(db), n, sb, ptr(dcb), 0, ptr(dc), n, sc, st())
+        y = dc.cpu().numpy()
+        assert np.array_equal(y[:, :m * n].reshape(batch, m, n), ref_batch) and (y[:, m * n:] == 7.0).all(), \
+            f"variant {v}: batch"
+        p, packed = layer.prepack_weights((batch, k, 1, n), dw)
+        dy = torch.full((batch, m, 1, n), 7.0, device=cuda)
+        N.call("osh_conv2d_add_f32", C.byref(p), ptr(dx), ptr(packed), ptr(drb), N.ACT_NONE, ptr(dres), ptr(dy), st())
+        assert np.array_equal(dy.cpu().numpy().reshape(batch, m, n), ref_conv), f"variant {v}: residual"
+
+
 def test_gemm_variants_row_bias_silu_and_column_scale(cuda, oracle, variant_reset):
     from onnxsharp_amd import native as N
     m, k, n = 128, 256, 640
