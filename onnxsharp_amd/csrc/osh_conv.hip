@@ -197,11 +197,11 @@ __global__ __launch_bounds__(256) void dw3_conv_kernel(osh_conv_params p, const 
 
 // K x K depthwise, dilation 1, stride S, left pad K / 2: four neighbouring
 // outputs of R rows a thread.  One output a thread spends most of its time on
-// index arithmetic and nine separate loads (4 x 128 x 112 x 112: 25.9 us, 2.0
+// index arithmetic and nine separate loads (4 x 128 x 112 x 112: 28.7 us, 1.8
 // TB/s); here a thread loads the 3 S + K columns under its strip once for all
 // four outputs (and, between its rows, once for both): the left halo one by
 // one, the rest, which starts at the strip's own column, 16 bytes at a time;
-// and it stores 16 bytes (12.5 us, 4.1 TB/s of the 4.75 a large copy reaches).
+// and it stores 16 bytes (13.5 us, 3.8 TB/s of the 4.95 a large copy reaches).
 // What lies outside the tensor loads as zero through
 // the buffer descriptor; taps off the map are skipped in the chain, as in
 // dw_conv_at.
@@ -970,9 +970,9 @@ static osh_status conv2d(const osh_conv_params *p, const float *d_x, const void 
         dim3 grid((unsigned)((total + 255) / 256));
         if (dws_eligible(p) && (p->kh == 5 || total >= DWS_MIN_OUTPUTS)) {
             // Rows a thread: more of them share loads, fewer of them keep more
-            // waves in flight.  Stride 1: 4 x 128 x 112 x 112 18.9, 15.2, 14.3
-            // us with 1, 2, 4 rows, 32 x 160 x 160 4.63, 4.28, 4.54, 64 x 80 x 80
-            // 3.46, 3.53, 4.42; stride 2 (rows share less): 4 x 128 x 112 x 112
+            // waves in flight.  Stride 1: 4 x 128 x 112 x 112 17.4, 14.6, 13.5
+            // us with 1, 2, 4 rows, 32 x 160 x 160 4.50, 4.16, 4.48, 64 x 80 x 80
+            // 3.42, 3.53, 4.41; stride 2 (rows share less): 4 x 128 x 112 x 112
             // 7.1, 7.2, 7.5.
             const int rows = p->sh == 2 || total < 800000 ? 1 : (p->kh == 5 || total < 4000000 ? 2 : 4);
             const long long threads = (long long)p->n * p->m * ((p->oh + rows - 1) / rows) * ((p->ow + 3) / 4);
@@ -1086,8 +1086,8 @@ static osh_status conv2d(const osh_conv_params *p, const float *d_x, const void 
             // one: 8 x 256 x 14 x 14 -> 256 (200 workgroups) 18.4 us (one block
             // 20.8), 2 x 64 x 13 x 74 -> 200 (231) 7.2 (8.0); 2 x 128 x 28 x 28 ->
             // 128 (100) 10.2 (8.4).  Past one workgroup a CU either can win: 2 x
-            // 40 x 70 x 24 -> 240 (424) 9.3 (10.8), 8 x 64 x 56 x 56 -> 64 (784) 21.4
-            // (21.3), 4 x 64 x 14 x 43 -> 200 (273) 10.4 (8.6).
+            // 40 x 70 x 24 -> 240 (424) 9.1 (10.4), 8 x 64 x 56 x 56 -> 64 (784) 20.7
+            // (20.5), 4 x 64 x 14 x 43 -> 200 (273) 10.3 (8.4).
             if (p->m > 16 && (tiles + 15) / 16 * ((p->m + 31) / 32) >= 5 * device_cus() / 8) OSH_WINO(2);
             else OSH_WINO(1);
             OSH_LAUNCH_CHECK("wino_f23_kernel");

@@ -25,10 +25,10 @@
 // groups ahead; the reads of a group are pinned between the MFMAs of the one
 // before (left alone the compiler sinks each to just before its use).
 //
-// Measured: the 7x7 stem above 20.3 us (46 TFLOP/s; the loop 12 us of it, whose
+// Measured: the 7x7 stem above 19.6 us (48 TFLOP/s; the loop 12 us of it, whose
 // 160 MFMAs a wave on CUs with four workgroups take 8.5, the rest the first
 // loads and 12.8 MB of output, which the workgroups reach together); 200 x 40 x
-// 40 -> 64 3x3 stride 2 138 -> 21.7; 512 x 14 x 14 -> 512 5x5 1618 -> 107.  Without
+// 40 -> 64 3x3 stride 2 137 -> 21.9; 512 x 14 x 14 -> 512 5x5 1628 -> 109.  Without
 // the operand reads the loop takes the same time.
 //
 // k past the last: W is -0 and the patch value +0 (a plane of zeros behind the

@@ -715,9 +715,10 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused_kernel(
                     sum = __builtin_amdgcn_sdot4(v, 0x01010101, sum, false);
                     dst[i * 256] = v;
                 }
-            } else {
+            } else {  // element by element, and no more than 8 k-steps where that is all
 #pragma unroll
                 for (int i = 0; i < KS; i++) {
+                    if (i == 8 && s0 + i >= ks) break;
                     const int kk = (s0 + i) * 32 + 4 * c8;
                     unsigned lm = 0;
 #pragma unroll
@@ -1150,7 +1151,7 @@ static osh_status launch_int8_gemm(int m, int k, int n, const int8_t *apk, const
     } while (0)
     // 64-row tiles (half the W traffic) where they still give 3 workgroups for
     // every 2 CUs, with two stages in flight so that more workgroups share a CU:
-    // 1028 x 1280 x 5120 26.2 us (32-row tiles 29.1); 669 x 352 x 2368 13.3 (12.8).
+    // 1028 x 1280 x 5120 25.2 us (32-row tiles 30.0); 669 x 352 x 2368 13.6 (13.3).
     if ((long long)((mt + 1) / 2) * nb >= 3LL * device_cus() / 2) OSH_I8_GEMM(2, 2);
     else OSH_I8_GEMM(1, 4);
 #undef OSH_I8_GEMM
@@ -1178,12 +1179,14 @@ static osh_status dqmm_run(int m, int k, int n, const float *d_a, const void *d_
                       (reinterpret_cast<uintptr_t>(d_a) & 15) == 0;
     const int variant = dqmm_variant();
     // Every 128-column block of the fused launch quantizes its rows again, which
-    // a separate quantize launch (about 4.3 us) ends: the two cross at about
-    // 1e9 products on ragged tiles (669 x 352 x 2368 11.4 us in two launches,
-    // 13.2 in three; 777 x 700 x 3000 22.3 and 17.7; 1028 x 1280 x 5120 44.4 and
-    // 26.2) and 4e9 on full ones (2048 x 512 x 2048 15.4 and 18.3; 1024 x 1024 x
-    // 4096 22.3 and 20.6).  At most 16 rows take the skinny kernel instead
-    // (16 x 2048 x 8192 14.3 us, 13.5 in three).
+    // a separate quantize launch (about 4.3 us) ends.  The two cross at 4e9
+    // products on full tiles (2048 x 512 x 2048 15.1 us in two launches, 18.3 in
+    // three; 1024 x 1024 x 4096 22.1 and 20.3) and between 0.5e9 and 2e9 on ragged
+    // ones: later with K % 4 == 0 (669 x 352 x 2368 11.7 and 13.3; 1256 x 812 x
+    // 1242 14.9 and 16.6; 777 x 700 x 3000 21.7 and 17.8; 1028 x 1280 x 5120 42.1
+    // and 25.2) than without, where the fused launch masks each element (268 x
+    // 1946 x 1907, just below the line, 25.1 and 15.5).  At most 16 rows take the
+    // skinny kernel instead (16 x 2048 x 8192 14.1 us, 14.2 in three).
     const double macs = (double)m * n * k;
     const bool three = variant == 1 || fblocks > 0x7fffffffLL || (m > 16 && macs > (full ? 4e9 : 1e9));
     osh_status r = run_minmax(d_a, total, sc, &nparts, st, three ? rownan : nullptr, three ? pad32(m) : 0);
