@@ -1004,8 +1004,9 @@ __global__ __launch_bounds__(64 * DQF_WAVES) void dqmm_fused16_kernel(
 // waves split K, k-step s to wave s % 4; the sums meet in LDS, exact in int32.
 // 256 / RT threads quantize each row, DQS_KS k-steps a pass; every wave's W
 // fragments of two passes (K = 2048) are in flight before the parameter
-// reduction.  Rows of the A tile past m are whatever LDS held: they reach only
-// output rows that do not exist; k-steps past the last meet zero W.
+// reduction.  Rows of the A tile past m, and k-steps past the last that are not
+// quantized, are whatever LDS held: the ones reach only output rows that do not
+// exist, the others meet zero W.
 constexpr int DQS_KS = 32;  // k-steps a pass
 constexpr int DQS_WS = DQS_KS / 4;
 
@@ -1064,6 +1065,8 @@ __global__ __launch_bounds__(256) void dqmm_skinny_kernel(
     auto pass = [&](i32x4 (&bb)[DQS_WS], int s0) {
 #pragma unroll
         for (int i = 0; i < RT; i++) {
+            // every 256 k: no more of them (9 x 90 x 88 8.6 us, so 7.0)
+            if (i && TPR * 4 * i % 256 == 0 && s0 * 32 + TPR * 4 * i >= k) break;
             const int kl = 4 * (c + TPR * i), kk = s0 * 32 + kl;
             unsigned lm = 0;
 #pragma unroll

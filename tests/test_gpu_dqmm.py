@@ -370,11 +370,16 @@ def _no_acc_case(cuda, oracle, m, k, n, noalloc, offset):
     (1, 1, 1, np.int8, 0, 2), (2, 31, 33, np.uint8, 0, 2), (3, 1024, 32, np.int8, 0, 2), (4, 1025, 31, np.uint8, 0, 2),
     (5, 2049, 65, np.int8, 0, 2), (8, 4097, 40, np.uint8, 0, 2), (9, 130, 513, np.int8, 0, 2),
     (16, 2050, 96, np.uint8, 0, 2),
+    # and rows quantized 256 k at a time: at, before and past the last
+    (3, 511, 70, np.int8, 0, 2), (5, 255, 40, np.uint8, 0, 2), (8, 257, 33, np.int8, 0, 2), (9, 90, 88, np.uint8, 0, 2),
+    (12, 256, 40, np.int8, 0, 2), (16, 1281, 64, np.uint8, 0, 2),
     # ragged tiles of the fused launch: one past a tile, k % 4 != 0, two and three passes
     (17, 36, 129, np.int8, 0, 2), (33, 513, 127, np.uint8, 0, 2), (65, 1100, 130, np.int8, 0, 2),
     # and at most 4, at most 8 and 9 or more k-steps
     (17, 127, 40, np.uint8, 0, 2), (33, 128, 33, np.int8, 0, 2), (40, 129, 130, np.int8, 0, 2),
     (20, 255, 70, np.int8, 0, 2), (64, 256, 129, np.uint8, 0, 2), (35, 257, 64, np.uint8, 0, 2),
+    # 8 and 9 k-steps left for the last pass
+    (40, 767, 33, np.int8, 0, 2), (20, 770, 129, np.uint8, 0, 2),
     # three launches, 32-row tiles: one and several stages, ragged in each direction
     (31, 33, 127, np.uint8, 1, 3), (33, 128, 129, np.int8, 1, 3), (65, 1157, 257, np.uint8, 1, 3),
     # 64-row tiles (enough workgroups), and the size rule's own choice of three launches
