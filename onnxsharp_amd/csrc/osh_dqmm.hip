@@ -204,49 +204,74 @@ struct Quad {
 };
 
 // MatMulInteger's activations: u8 (a - 128) or s8 (a) into the s8 a'' of the
-// MFMA layout.  A wave takes DQ_MF fragments (32 rows x 32 k) of one row tile:
-// lane l loads 16 consecutive bytes of row l & 31, k half l >> 5 -- with one
-// 16-byte load where every row is 16-byte aligned -- and stores them at l * 16.
+// MFMA layout.  A wave takes one fragment (32 rows x 32 k; four a wave were
+// slower at every size: 1000 x 1000 x 64, both launches, 8.4 us against 7.5, 8192 x
+// 2048 x 64 18.8 against 17.6).
+// VEC, every row 16-byte aligned: lane l loads 16 consecutive bytes of row l &
+// 31, k half l >> 5, and stores them at l * 16.  Else lane l takes the four
+// bytes at k = 4 (l % 8) of row l / 8 + 8 i, with one 4-byte load at whatever
+// address; one that would pass the end of A starts earlier and is shifted.  No
+// load waits for another (16 guarded bytes a lane, in four fragments: 318 x 115 x
+// 519 11.6 us, so 5.7; 9 x 121 x 16 10.1, so 4.6).
 // Block 0 publishes alpha = (u8 ? 128 : 0) - a_zp so that a - a_zp = a'' +
 // alpha; no row is NaN.
-constexpr int DQ_MF = 4;
-
+template <bool VEC>
 __global__ __launch_bounds__(DQ_THREADS) void mmi_pack_a_kernel(const uint8_t *__restrict__ a, int m, int k,
                                                                  int a_signed, int a_zp, DqScratch *__restrict__ sc,
                                                                  int *__restrict__ rownan, int8_t *__restrict__ apk) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ks = pad32(k) / 32, nch = (ks + DQ_MF - 1) / DQ_MF;
+    const int ks = pad32(k) / 32;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         sc->alpha = (a_signed ? 0 : 128) - a_zp;
         sc->scale = 1.0f;
         sc->zp = a_zp;
     }
-    const int w = blockIdx.x * (DQ_THREADS / 64) + wave;
-    const int mt = w / nch, s0 = w % nch * DQ_MF;
-    if (mt * 32 >= m) return;
-    const int row = mt * 32 + (lane & 31);
-    const bool live = row < m;
-    if (s0 == 0 && lane < 32) rownan[row] = 0;
-    const uint8_t *src = a + (long long)(live ? row : 0) * k;
-    const bool vec = (k & 15) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+    const long long w = (long long)blockIdx.x * (DQ_THREADS / 64) + wave;
+    const int mt = (int)(w / ks), s = (int)(w % ks);
+    if ((long long)mt * 32 >= m) return;
+    if (s == 0 && lane < 32) rownan[mt * 32 + lane] = 0;
     const unsigned flip = a_signed ? 0u : 0x80808080u;  // u8 - 128, byte by byte
+    int8_t *dst = apk + w * 1024;
+    if constexpr (VEC) {
+        const int row = mt * 32 + (lane & 31), kk = s * 32 + 16 * (lane >> 5);
+        const bool live = row < m && kk < k;
+        i32x4 v = *reinterpret_cast<const i32x4 *>(a + (live ? (long long)row * k + kk : 0));
 #pragma unroll
-    for (int f = 0; f < DQ_MF; f++) {
-        const int s = s0 + f, kk = s * 32 + 16 * (lane >> 5);
-        i32x4 v = {};  // padding rows and columns carry a'' = 0
-        if (live && vec) {
-            if (kk < k) {
-                v = *reinterpret_cast<const i32x4 *>(src + kk);
+        for (int e = 0; e < 4; e++) v[e] = live ? v[e] ^ (int)flip : 0;  // padding rows and columns carry a'' = 0
+        *reinterpret_cast<i32x4 *>(dst + lane * 16) = v;
+    } else {
+        const int r8 = lane >> 3, c8 = lane & 7, kk = s * 32 + 4 * c8;
+        const long long total = (long long)m * k, last = total < 4 ? 0 : total - 4;
+        unsigned v[4];
+        int past[4];
+        auto each = [&](auto load) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] ^= (int)flip;
+            for (int i = 0; i < 4; i++) {
+                const long long at = (long long)(mt * 32 + 8 * i + r8) * k + kk;
+                const long long from = at < last ? at : last;
+                past[i] = at - from < 3 ? (int)(at - from) : 3;  // more only past the row
+                v[i] = load(a + from);
             }
-        } else if (live) {
-#pragma unroll
-            for (int e = 0; e < 16; e++)
-                if (kk + e < k)
-                    v[e >> 2] |= (int)(((unsigned)src[kk + e] ^ (flip & 0xffu)) << (8 * (e & 3)));
+        };
+        if (total >= 4) {
+            each([](const uint8_t *src) {
+                unsigned u;
+                __builtin_memcpy(&u, src, 4);
+                return u;
+            });
+        } else {  // all of an A of 1 to 3 bytes
+            unsigned u = 0;
+            for (int e = 0; e < total; e++) u |= (unsigned)a[e] << (8 * e);
+            each([&](const uint8_t *) { return u; });
         }
-        if (s < ks) *reinterpret_cast<i32x4 *>(apk + (((long long)mt * ks + s) * 64 + lane) * 16) = v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = mt * 32 + 8 * i + r8, left = row < m ? k - kk : 0;
+            const unsigned mask = left >= 4 ? ~0u : (left > 0 ? (1u << (8 * left)) - 1 : 0u);
+            // lane slot (row & 31) + 32 * (c8 >> 2); byte 4 (c8 & 3)
+            reinterpret_cast<unsigned *>(dst)[(8 * i + r8 + 32 * (c8 >> 2)) * 4 + (c8 & 3)] =
+                ((v[i] >> (8 * past[i])) ^ flip) & mask;
+        }
     }
 }
 
@@ -329,9 +354,10 @@ __device__ __forceinline__ ColOperands load_column(int j, int n, const int *__re
 // ends the prefetch and pads the last stage without a branch.  Row sums of a''
 // come from the staged registers (v_dot4).
 //
-// Bound by LDS and L1 traffic and, at the ends, the first loads and the output
-// stores: 1028 x 1280 x 5120 takes 18.5 us here (13.5 G int-ops, 727 TOP/s; 4
-// us of it stores, 6 the first loads and the epilogue), 512 x 512 x 2048 4.8.
+// Bound by what the L2s deliver and, at the ends, the first loads and the output
+// stores: 1028 x 1280 x 5120 takes 16.3 us here (13.5 G int-ops, 827 TOP/s), in
+// which the workgroups read 167 MB of fragments from L2 (10 TB/s) while LDS is
+// active 15% of the time and the int8 units 17%; 512 x 512 x 2048 4.8.
 constexpr int DQG_KS = 4;
 enum { DQG_FLOAT = 1, DQG_ACC = 2 };  // which outputs a launch writes
 
@@ -417,6 +443,7 @@ __global__ __launch_bounds__(256, 2) void dqmm_gemm_kernel(int m, int k, int n, 
                 for (int t = 0; t < TM; t++)
                     acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[(t * DQG_KS + kk) * 64], r[u].b[kk], acc[t], 0,
                                                                    0, 0);
+            if (st + u + 1 >= nst) break;
             load(r[u], st + u + SETS);
             stage(r[(u + 1) % SETS], (u + 1) & 1);
             add_rows(r[(u + 1) % SETS]);
@@ -1156,6 +1183,8 @@ static osh_status launch_int8_gemm(int m, int k, int n, const int8_t *apk, const
     // every 2 CUs, with two stages in flight so that more workgroups share a CU:
     // 1028 x 1280 x 5120 25.2 us (32-row tiles 30.0); 669 x 352 x 2368 13.6 (13.3).
     if ((long long)((mt + 1) / 2) * nb >= 3LL * device_cus() / 2) OSH_I8_GEMM(2, 2);
+    // of which no more in flight than there are (1 x 18 x 3094 5.05 us, with four 5.24)
+    else if (k <= 2 * 32 * DQG_KS) OSH_I8_GEMM(1, 2);
     else OSH_I8_GEMM(1, 4);
 #undef OSH_I8_GEMM
 #undef OSH_I8_GEMM_OUT
@@ -1391,11 +1420,17 @@ OSH_API osh_status osh_matmul_integer(int m, int k, int n, const void *d_a, int 
     DqScratch *sc = static_cast<DqScratch *>(d_scratch);
     int *rownan = reinterpret_cast<int *>(sc + 1);  // the second mpad ints of the layout are spare
     int8_t *apk = reinterpret_cast<int8_t *>(rownan + 2 * pad32(m));
-    const long long waves = (long long)(pad32(m) / 32) * ((pad32(k) / 32 + DQ_MF - 1) / DQ_MF);
-    const long long pblocks = (waves + DQ_THREADS / 64 - 1) / (DQ_THREADS / 64);
+    const uint8_t *a = static_cast<const uint8_t *>(d_a);
+    const bool vec = k % 16 == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+    const long long frags = (long long)(pad32(m) / 32) * (pad32(k) / 32);
+    const long long pblocks = (frags + DQ_THREADS / 64 - 1) / (DQ_THREADS / 64);
     if (pblocks > 0x7fffffffLL) return fail(OSH_E_UNSUPPORTED, "MatMulInteger: m too large");
-    OSH_LAUNCH(mmi_pack_a_kernel, dim3((unsigned)pblocks), dim3(DQ_THREADS), 0, st,
-               static_cast<const uint8_t *>(d_a), m, k, a_signed, a_zp, sc, rownan, apk);
+#define OSH_MMI_PACK(VEC)                                                                                      \
+    OSH_LAUNCH(mmi_pack_a_kernel<VEC>, dim3((unsigned)pblocks), dim3(DQ_THREADS), 0, st, a, m, k, a_signed, \
+               a_zp, sc, rownan, apk)
+    if (vec) OSH_MMI_PACK(true);
+    else OSH_MMI_PACK(false);
+#undef OSH_MMI_PACK
     OSH_LAUNCH_CHECK("mmi_pack_a_kernel");
     const int8_t *frag = static_cast<const int8_t *>(d_wpacked);
     const int *colsum = reinterpret_cast<const int *>(frag + (size_t)pad32(n) * pad32(k));

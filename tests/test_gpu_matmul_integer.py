@@ -58,6 +58,29 @@ def test_matmul_integer_parity(cuda, oracle, m, k, n, adt, azp, bdt, bzp):
     assert np.array_equal(y, ref), f"max |d| {np.abs(y.astype(np.int64) - ref).max()}"
 
 
+@pytest.mark.parametrize("m,k,n,offset,adt", [
+    (1, 1, 5, 0, "u8"), (1, 2, 33, 1, "s8"), (3, 1, 7, 2, "u8"), (1, 4, 9, 3, "s8"),  # A of 1 to 4 bytes
+    (2, 31, 40, 1, "u8"), (33, 33, 65, 3, "s8"), (32, 64, 129, 0, "u8"), (32, 64, 129, 8, "u8"),  # odd rows, odd bases
+    (65, 130, 33, 2, "s8"), (31, 257, 70, 0, "u8"), (5, 288, 40, 0, "s8"),  # two stages and one k-step more
+    (2047, 2050, 40, 1, "u8"), (1028, 96, 6500, 0, "u8"),  # many workgroups; 64-row tiles
+])
+def test_matmul_integer_any_address(cuda, oracle, m, k, n, offset, adt):
+    """Activations at every byte offset and row length: the bytes before and
+    after them (all ones) reach no sum."""
+    import torch
+    from onnxsharp_amd.layers import MatMulIntegerLayer
+    print(f"matmulinteger m={m} k={k} n={n} offset={offset} A {adt}", flush=True)
+    dt, lo, hi = (np.uint8, 0, 255) if adt == "u8" else (np.int8, -128, 127)
+    a = synth.randint(m + k, (m, k), lo, hi, dt)
+    b = synth.randint(n + k, (k, n), -128, 127, np.int8)
+    buf = torch.full((offset + m * k + 64,), -1, dtype=torch.int8, device=cuda)
+    buf[offset:offset + m * k] = _t(a.view(np.int8).reshape(-1), cuda)
+    da = buf[offset:offset + m * k].view(torch.uint8 if adt == "u8" else torch.int8).view(m, k)
+    assert da.is_contiguous() and da.data_ptr() == buf.data_ptr() + offset
+    y = MatMulIntegerLayer().forward(da, _t(b, cuda), [7]).cpu().numpy()
+    assert np.array_equal(y, oracle.matmul_integer(a, b, 7))
+
+
 def test_matmul_integer_batch1_3d_and_errors(cuda, oracle):
     from onnxsharp_amd import native as N
     from onnxsharp_amd.layers import MatMulIntegerLayer
