@@ -355,9 +355,9 @@ __device__ __forceinline__ ColOperands load_column(int j, int n, const int *__re
 // come from the staged registers (v_dot4).
 //
 // Bound by what the L2s deliver and, at the ends, the first loads and the output
-// stores: 1028 x 1280 x 5120 takes 16.3 us here (13.5 G int-ops, 827 TOP/s), in
-// which the workgroups read 167 MB of fragments from L2 (10 TB/s) while LDS is
-// active 15% of the time and the int8 units 17%; 512 x 512 x 2048 4.8.
+// stores: 1028 x 1280 x 5120 takes 15.7 us here (13.5 G int-ops, 858 TOP/s), in
+// which the workgroups read 167 MB of fragments from L2 (10.6 TB/s) while LDS is
+// active 15% of the time and the int8 units 18%; 512 x 512 x 2048 4.8.
 constexpr int DQG_KS = 4;
 enum { DQG_FLOAT = 1, DQG_ACC = 2 };  // which outputs a launch writes
 

@@ -28,13 +28,13 @@
 // [comp][oc][tile] and each thread transforms one (oc, tile) to its 2x2
 // outputs, stored two at a time.
 //
-// Bound by what the L2s deliver: 8 x 64 x 56 x 56 -> 64 with a residual reads
-// 215 MB through L1 with one output block a workgroup (weights once per 16
-// tiles, patches once per 16 channels), 160 with two, at about 15 TB/s: 21.3 us
-// with either (33.5 with patch loads and stores one guarded value at a time; 24.1
-// and 22.5 when the last chunks were not yet apart, which showed workgroups of 32
-// tiles, weights shared through L1, slower by 5-10%, all 16 components x 32 x 32
-// in four waves by 40% (registers), patches two chunks ahead no change).
+// Bound by waiting: at 8 x 64 x 56 x 56 -> 64 with a residual (21.3 us; 33.5 with
+// patch loads and stores one guarded value at a time) the waves wait for 48% of
+// their cycles, at each chunk's barrier and for the loads behind it, with the MFMAs
+// 24% busy, vector issue 19%, LDS 14%, L2 reads 8 TB/s.  One output block a
+// workgroup reads a third more through L1 and takes the same time.  Slower:
+// workgroups of 32 tiles, weights shared through L1 (5-10%); all 16 components x 32
+// x 32 in four waves (40%: registers); patches two chunks ahead, no change.
 #pragma once
 
 #include "osh_common.h"
