@@ -33,6 +33,8 @@ static const G16Variant kG16[] = {
     {1, 1, 2, 64},  // 10: 16 x 32, 64-k chunks
 };
 constexpr int kG16Count = sizeof(kG16) / sizeof(kG16[0]);
+// Waves a SIMD holds of each (the compiler's occupancy, by registers).
+static const int kG16Resident[kG16Count] = {7, 5, 4, 3, 3, 2, 2, 2, 2, 3, 3};
 
 }  // namespace osh
 
@@ -51,35 +53,37 @@ static bool g16_fits(const IgemmArgs &a) {
     return a.K >= 1 && ((a.M - 1LL) * a.lda + kmax) * 4 < (1LL << 31) && (kmax * a.ldb + a.N + 64) * 4 < (1LL << 31);
 }
 
-// Predicted time of a wave tile, in cycles, less what all tiles share.  A wave's
-// chunk takes its MFMAs (32 cycles each, 90 more a chunk) or, where those are
-// fewer, one trip past L2 (loads are one chunk ahead).  64-k chunks pay only for
-// such trips, of small waves: their MFMAs are no fewer, their prologue is longer.
+// Predicted time of a wave tile, in cycles.  A wave's chunk takes its MFMAs (32
+// cycles each) or, where those are fewer, one trip past L2 (loads are one chunk
+// ahead).  64-k chunks pay only for such trips, of small waves: their MFMAs are no
+// fewer, their prologue is longer.
 // Whether the operands (A and B together) come from past L2 is put at 6 MB.  What
 // a program that multiplies by other weights in between sees is the cold side: 7 x
 // 480 x 3840 8.6 us with 16 x 16 tiles of 32 k, 7.1 of 64 k, 14 x 3584 x 480 41.7
 // and 25.9; the same operands again and again, in L2, take 5.7 and 6.5, 20.6 and 25.
-// Further waves of a SIMD add their MFMAs (its pipe is full by then, so a little
-// less than 32 cycles each), address and LDS work, prologue and epilogue (more
-// for two row blocks); their number is half way between the average and the
-// fullest SIMD's, since workgroups that end early make room for others.
+// A SIMD takes its waves in rounds of as many as its registers hold (kG16Resident),
+// and the fullest SIMD counts.  Of a round, the first wave costs its whole time;
+// the others fill the gaps of its MFMAs and add what is left of theirs, address and
+// LDS work, prologue and epilogue, more for two row blocks.
 // Workgroups of four waves fill the chip by fours, so slots count, not tiles
 // (of fewer row tiles the idle waves leave at once).
-// Fitted to 979 products and batches (m 1-4096, k 32-4096, n 32-8192), each with
-// its operands in L2 and out of it: on average 0.9% and 2.1% above the best tile
-// (an earlier fit with hardly a term for the fullest SIMD 1.6% and 2.8%, its 64-k
-// tiles among several waves a SIMD up to 36% slower: 1946 x 448 x 2560 58.1 ->
-// 45.5 us, 14 of 436 x 128 x 436 19.2 -> 14.2).
-static double g16_cost(const IgemmArgs &a, int zcount, const G16Variant &v, int cus) {
+// Fitted to 2517 products and batches (m 1-4096, k 32-4096, n 32-8192), each with
+// its operands in L2 and out of it: on average 0.8% and 1.8% above the best tile.
+// With waves in place of rounds 1.3% and 2.3% (1009 x 64 x 3808 13.7 -> 11.4
+// us, 2908 x 1120 x 2912 177 -> 160); with hardly a term for the fullest SIMD before
+// that, 64-k tiles among several waves a SIMD were up to 36% slower (1946 x 448 x
+// 2560 58.1 -> 45.5 us, 14 of 436 x 128 x 436 19.2 -> 14.2).
+static double g16_cost(const IgemmArgs &a, int zcount, int variant, int cus) {
+    const G16Variant &v = kG16[variant];
     const int tiles_m = ceil_div(a.M, 16 * v.tm), waves = std::min(tiles_m, 4);
     const double slots = (double)ceil_div(tiles_m, waves) * waves * ceil_div(a.N, 16 * v.bv * v.tn) * zcount;
     const double u = (double)v.tm * v.tn * v.bv, k32 = v.kc / 32.0;
     const bool far = 4.0 * zcount * ((double)a.M * a.K + (double)a.K * a.N) > 6e6;
-    const double chunks = ceil_div(a.K, v.kc), trip = v.kc == 32 ? (far ? 700 : 0) : (far ? 850 : 3000);
-    const double per_simd = slots / (4.0 * cus);
-    const double more = std::max(0.0, 0.5 * std::ceil(per_simd) + 0.5 * per_simd - 1.0);
-    return 1500 * u + (v.kc == 64 ? 3500 : 0) + chunks * std::max(trip, 90 + 256 * u * k32) +
-           more * (chunks * k32 * (230 * u + 450) + 1000 * u + 300 + 4500 * (v.tm - 1));
+    const double chunks = ceil_div(a.K, v.kc), trip = v.kc == 32 ? (far ? 920 : 0) : (far ? 760 : 3000);
+    const double fullest = std::ceil(slots / (4.0 * cus)), rounds = std::ceil(fullest / kG16Resident[variant]);
+    const double first = 8000 + 1700 * u + (v.kc == 64 ? 6700 : 0) + chunks * std::max(trip, 256 * u * k32);
+    const double other = chunks * k32 * (100 * u + 420) + 900 * u + 1500 + 5200 * (v.tm - 1);
+    return rounds * std::max(first, other) + (fullest - rounds) * other;
 }
 
 template <int TM, int TN, int BV, int KC>
@@ -106,7 +110,7 @@ static bool launch_gemm16(const IgemmArgs &a, int zcount, int act, hipStream_t s
         double bc = 0;
         for (int i = 0; i < kG16Count; i++) {
             if (a.N < kG16[i].bv) continue;
-            const double c = g16_cost(a, zcount, kG16[i], cus);
+            const double c = g16_cost(a, zcount, i, cus);
             if (best < 0 || c < bc) best = i, bc = c;
         }
     }
